@@ -43,6 +43,7 @@ __device__ void jacobi_work(void* token);
 #include <vector>
 
 #include "jacobi2d_internal.h"
+#include "pipeline.h"
 
 #define LEFT 0
 #define RIGHT 1
@@ -73,6 +74,7 @@ struct JacobiDesc {
   int overlap;            // sweep edges first, send, then the interior
   uint64_t* recv_ticks;   // per chare: ticks inside recv_ghosts (unpack)
   int depth;              // halo depth = sweeps per exchange (1 .. 16)
+  double ring;            // the value of the grid's ring
   int halo_copy;          // 1: halos staged and copied by invoke (else the
                           // sweep writes them into the messages in place)
 };
@@ -458,6 +460,36 @@ __device__ void sweepD_dispatch(int steps, const double* in, double* out,
 #undef CHM_CASED
 }
 
+// Sixteen fused sweeps of the whole block (halos sixteen deep) by groups of
+// four waves (pipeline.h): every full round but the last of a solve, unless
+// the caller asked for bands of the window pass.  16384^2 x 1000, 16 x 16
+// chares: 118-119 -> 90-91 ms per solve; 4096^2 x 200, 8 x 8 chares:
+// 10.9 -> 6.4 ms.  Other depths and the last round (its residual) run the
+// window pass.
+__device__ __noinline__ void chare_pipe(const double* in, double* out,
+                                        int64_t P, int bw, int bh,
+                                        RingSides rs) {
+  __shared__ PipeLds lds[CHARMING_PE_THREADS / 64 / kPipeWaves];
+  PipeBlock b;
+  b.in = wuni(in);
+  b.out = wuni(out);
+  b.pitch = wuni(P);
+  b.cols.c0 = b.r0 = 1;
+  b.cols.c1 = wuni(bw) + 1;
+  b.r1 = wuni(bh) + 1;
+  b.top = wuni((int)rs.top) ? 0 : kNoRing;
+  b.bottom = wuni((int)rs.bottom) ? b.r1 : kNoRing;
+  b.cols.left = wuni((int)rs.left) ? 0 : kNoRing;
+  b.cols.right = wuni((int)rs.right) ? b.cols.c1 : kNoRing;
+  b.cols.flat = true;
+  b.ring = g_jdesc.ring;
+  b.lo_col = b.lo_row = 1 - kHaloRows;
+  b.hi_col = b.cols.c1 - 1 + kHaloRows;
+  b.hi_row = b.r1 - 1 + kHaloRows;
+  pipe_block<CHARMING_PE_THREADS, kHaloRows / kPipeWaves, false>(b, lds,
+                                                                 nullptr);
+}
+
 // The whole workgroup: the outgoing edges of the array g, D deep, into the
 // messages' payloads (layout of EdgeOut2: top = rows 1..D, bottom = rows
 // bh-D+1..bh, w each; left = columns 1..D, right = columns bw-D+1..bw, h
@@ -635,6 +667,42 @@ __device__ void Block::send_boundaries() {
   }
 }
 
+// The whole workgroup copies ni x nj cells from src to dst (rows of sp and
+// dp elements), kPutBatch loads in flight per lane (a chare of 1024^2 puts
+// its edges in 42 us a round; one load at a time made a 16384^2 x 1000 solve
+// 2.2 ms longer).
+constexpr int kPutBatch = 8;
+template <class V>
+__device__ inline void copy_block_as(const double* src, int64_t sp,
+                                     double* dst, int64_t dp, int ni, int nj) {
+  typedef __attribute__((address_space(1))) const V gcv;
+  typedef __attribute__((address_space(1))) V gv;
+  constexpr int kN = (int)(sizeof(V) / sizeof(double));
+  const int per = nj / kN, total = ni * per, W = blockDim.x;
+  for (int e0 = threadIdx.x; e0 < total; e0 += kPutBatch * W) {
+    V v[kPutBatch];
+#pragma unroll
+    for (int x = 0; x < kPutBatch; x++) {
+      const int e = min(e0 + x * W, total - 1), i = e / per, j = e - i * per;
+      v[x] = *(gcv*)(src + i * sp + j * kN);
+    }
+#pragma unroll
+    for (int x = 0; x < kPutBatch; x++) {
+      const int e = e0 + x * W, i = e / per, j = e - i * per;
+      if (e < total) *(gv*)(dst + i * dp + j * kN) = v[x];
+    }
+  }
+}
+// (pairs of cells where both sides allow it: rows of an even number of
+// elements throughout, so the first cells decide)
+__device__ inline void copy_block(const double* src, int64_t sp, double* dst,
+                                  int64_t dp, int ni, int nj) {
+  if ((((uintptr_t)src | (uintptr_t)dst) & 15) == 0 && (nj & 1) == 0)
+    copy_block_as<v2d>(src, sp, dst, dp, ni, nj);
+  else
+    copy_block_as<double>(src, sp, dst, dp, ni, nj);
+}
+
 // Deep rounds with zero-copy halos: the workgroup writes the new grid's
 // edges, D deep, and its (D-1) x (D-1) corner blocks straight into the halo
 // of each neighbour's array of the same parity (the one its next round
@@ -643,11 +711,13 @@ __device__ void Block::send_boundaries() {
 // only the interior of this one, and its previous round (which read this
 // halo) has ended, or this chare could not have run its own.  The messages
 // that follow only notify (slot word 1 = 1: placed).  g was just written by
-// other waves, partly with streaming stores: loads at agent scope.
+// other waves, partly with streaming stores: the fence drops what the CU's
+// L1 holds of it.
 __device__ void Block::put_edges(const double* g, int D, int parity) {
   const JacobiDesc& d = g_jdesc;
   const int bw = block_width, bh = block_height;
   const int64_t P = pitch;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   for (int k = 0; k < N_NEIGHBORS; k++) {
     const int n = neighbor_index[k];
     if (n < 0) continue;
@@ -685,14 +755,8 @@ __device__ void Block::put_edges(const double* g, int D, int parity) {
         ni = nj = D - 1;
         break;
     }
-    for (int e = threadIdx.x; e < ni * nj; e += blockDim.x) {
-      const int i = e / nj, j = e % nj;
-      const uint64_t v = __hip_atomic_load(
-          (const uint64_t*)(g + (int64_t)(si0 + i) * P + kColOff + sj0 + j),
-          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      t[(int64_t)(di0 + i) * PN + kColOff + dj0 + j] =
-          __longlong_as_double((long long)v);
-    }
+    copy_block(g + (int64_t)si0 * P + kColOff + sj0, P,
+               t + (int64_t)di0 * PN + kColOff + dj0, PN, ni, nj);
   }
 }
 
@@ -817,7 +881,10 @@ __device__ void Block::update() {
                             neighbor_index[LEFT] < 0,
                             neighbor_index[RIGHT] < 0};
       if (steps >= 3) {
-        sweepD_dispatch(steps, t, nt, P, bw, bh, last, rs);
+        if (steps == kHaloRows && !last && g_jdesc.tune_band == 0)
+          chare_pipe(t, nt, P, bw, bh, rs);
+        else
+          sweepD_dispatch(steps, t, nt, P, bw, bh, last, rs);
         if (!last) {
           __syncthreads();
           if (put)
@@ -1024,6 +1091,7 @@ int persistent_create(Handle* h) {
   d.cr = cr;
   d.cc = cc;
   d.iters = h->prob.iters;
+  d.ring = h->prob.init_mode == CHM_INIT_REFERENCE ? 10.0 : h->prob.boundary;
   ps->n_chares = cr * cc;
   // the last chare row/column is the largest
   const ChareGeom gmax = chare_geom(h->W, h->H, cr, cc, cr * cc - 1);

@@ -238,3 +238,24 @@ def test_phase_times_per_chare(cam):
         j.solve()
         with pytest.raises(cam.ChmError):
             j.chare_phases()
+
+
+@pytest.mark.parametrize("W,H,cr,cc", [
+    # one chare, both ring columns in a window, at and past its width
+    (192, 33, 1, 1), (193, 16, 1, 1), (320, 17, 1, 1), (321, 40, 1, 1),
+    (576, 31, 1, 1), (577, 64, 1, 1), (1121, 50, 1, 1),
+    # a ring column at either end, odd and even widths; windows with none
+    (2 * 176, 100, 2, 2), (2 * 177, 99, 2, 2), (3 * 160, 64, 1, 3),
+    (3 * 161, 48, 3, 3), (2 * 560, 37, 1, 2), (2 * 561, 32, 2, 2),
+    (3 * 1024, 24, 1, 3), (3 * 1025, 19, 1, 3)])
+def test_wave_group_windows(cam, W, H, cr, cc):
+    # full rounds of sixteen sweeps shared by groups of four waves, at the
+    # edges of their windows (192, 320, 576 columns), and a last partial round
+    iters = 16 * 3 + 1
+    ref, res = O.jacobi_run(W, H, iters, seed=W + H, boundary=0.3)
+    with cam.Jacobi2D(W, H, iters, form="persistent", seed=W + H,
+                      boundary=0.3, chares=(cr, cc)) as j:
+        r = j.solve()
+        g = j.grid()
+    assert np.array_equal(g, ref)
+    assert r.residual == res and r.hash == O.grid_hash(ref)
