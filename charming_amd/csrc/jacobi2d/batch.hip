@@ -28,6 +28,7 @@
 
 #include "engine_dev.h"
 #include "jacobi2d_internal.h"
+#include "pipeline.h"
 
 namespace chm {
 namespace eng {
@@ -176,6 +177,9 @@ __device__ void do_round2(const Request& r, const TileGeom& g, int src,
 constexpr int kDeep = 8;       // fixed sweep counts, 1024-thread workgroups
 constexpr int kDeepWide = 16;  // fixed sweep counts, up to 512 threads
 constexpr int kWideRing = 6;   // input-ring slots of the sixteen-deep pass
+// engines whose full rounds run as groups of waves (pipeline.h): two groups,
+// one workgroup per CU
+constexpr int kPipeThreads = 512;
 
 __host__ __device__ constexpr int deep_for_threads(int threads) {
   return threads <= 512 ? kDeepWide : kDeep;
@@ -215,6 +219,36 @@ __device__ __noinline__ void do_round_deep(const double* in, double* out,
     pos += len;
   }
   if (RES) add_residual(res_slot + 2, acc);
+}
+
+// 4 NST sweeps of a tile by groups of four waves (pipeline.h).  SUM: the
+// FP64 sum of the last sweep's squared changes is added to *sum.  A 544 x 544
+// tile takes sixteen sweeps in 0.28 ms on a busy card, about 0.45 with
+// do_round_deep.
+template <int T, int NST, bool SUM>
+__device__ __noinline__ void do_round_pipe(const Request* rp, int r0, int r1,
+                                           int c0, int c1, int src, int dst,
+                                           double* sum) {
+  constexpr int D = jac::kPipeWaves * NST;
+  jac::PipeBlock b;
+  b.in = uni(arr(*rp, src));
+  b.out = uni(arr(*rp, dst));
+  b.pitch = uni(rp->pitch);
+  const int W = uni(rp->W), H = uni(rp->H);
+  b.cols.c0 = uni(c0);
+  b.cols.c1 = uni(c1);
+  b.cols.left = 0;
+  b.cols.right = W + 1;
+  b.cols.flat = true;
+  b.r0 = uni(r0);
+  b.r1 = uni(r1);
+  b.top = 0;
+  b.bottom = H + 1;
+  b.lo_col = b.lo_row = 1 - D;
+  b.hi_col = W + D;
+  b.hi_row = H + D;
+  b.ring = uni(rp->init_mode) == CHM_INIT_REFERENCE ? 10.0 : uni(rp->boundary);
+  jac::pipe_block<T, NST, SUM>(b, uni(sum));
 }
 
 // Rounds of tolerance problems: 3 .. D sweeps of a tile in one pass (D -
@@ -371,6 +405,36 @@ __device__ inline bool filtered_round(const Request& r, int rr) {
   return r.tol2 >= 0 && r.depth >= 3 && rr > 0 && rr + 1 < r.rounds;
 }
 
+// Rounds that run as groups of waves: windows start on odd columns, so every
+// tile of the problem has to.
+__device__ inline bool pipe_tiles(const Request& r) {
+  return (r.bs & 1) == 0 || r.tc == 1;
+}
+
+// Thread 0: the same for a filtered round run as groups of waves, which sums
+// the last sweep only.  With D_j = u_j - u_{j-1}, D_{j+1} = 0.2 A D_j + e:
+// A (a cell and its four neighbours) is symmetric with norm at most 5, and e
+// is what two sweeps round, at most 2 x 3.8 x 2^-53 M a cell, M the largest
+// |u|.  So |D_j| >= |D_n| - n E over the N cells for every earlier sweep,
+// E = sqrt(N) 2^-48 M holding e four times over (0.2 is rounded up, which
+// grows |u| and |D_j| by 2^-53 a sweep), and one sum of two operations per
+// cell and round replaces n of three.  With it the exact S_j, which truncates
+// less than 1 a cell as above, exceeds 2^56 (|D_n| - n E)^2 - N.
+__device__ bool pipe_may_stop(Prob& p, const Request& r, int sk) {
+  const double thr = r.tol2 * u128d(ald(&p.s0[0]), ald(&p.s0[1]));
+  if (!(thr < 0x1.0p62)) return true;
+  const double n = (double)r.W * (double)r.H;
+  const double a =
+      __longlong_as_double((long long)ald((uint64_t*)&p.resd[sk][0]));
+  const double m = r.init_mode == CHM_INIT_REFERENCE
+                       ? 10.0
+                       : fmax(1.0, fabs(r.boundary));
+  const double x = sqrt(a) * (1.0 - 0x1.0p-20) -
+                   (double)r.depth * sqrt(n) * m * 0x1.0p-48;
+  return !(x > 0.0 &&
+           x * x * 0x1.0p56 * (1.0 - 0x1.0p-20) - n > thr * (1.0 + 0x1.0p-20));
+}
+
 // Thread 0: whether a filtered round may hold the stop.  The exact residual
 // of sweep j is S_j = sum floor(fl(d^2) 2^56) over the cells (saturating at
 // 2^64 - 1), so S_j >= 2^56 T_j - N with T_j = sum fl(d^2) when no term
@@ -469,6 +533,7 @@ __device__ int decide_exact(Prob& p, const Request& r, int rr, int sk) {
 // decision comes before the release of round rr+1 (engine_kernel), so
 // decisions are made in order and round rr's input (array rr % 3) is intact
 // when it is decided even if round rr+1 is running.
+template <int T>
 __device__ int decide_round(Prob& p, const Request& r, int rr) {
   const bool tol = r.tol2 >= 0;
   const bool last = rr + 1 == r.rounds;
@@ -479,7 +544,9 @@ __device__ int decide_round(Prob& p, const Request& r, int rr) {
   // every tile has finished round rr: its residuals are complete
   if (ald(&p.state) != 0) return 0;  // stopped on the previous round
   if (filtered_round(r, rr)) {
-    if (filter_may_stop(p, r, sk, r.depth)) {
+    const bool pipe =
+        T == kPipeThreads && r.depth == kDeepTolWide && pipe_tiles(r);
+    if (pipe ? pipe_may_stop(p, r, sk) : filter_may_stop(p, r, sk, r.depth)) {
       ast(&p.resid_round, (uint32_t)rr);
       ast(&p.resid_tiles, 0u);
       ast(&p.state, 5u);
@@ -669,15 +736,23 @@ __device__ int find_work(const EngineDesc& E, uint32_t* task, uint64_t* req,
 
 // Round rr of a tile: `depth` fused sweeps (or what is left in the last
 // round), with the residuals the problem needs.
+// (rl: the request in LDS)
 template <int T, int NC, int U>
-__device__ void run_round(const Request& r, const TileGeom& g, int rr,
-                          Prob& p) {
+__device__ void run_round(const Request& r, const Request* rl,
+                          const TileGeom& g, int rr, Prob& p) {
   const bool tol = r.tol2 >= 0;
   const bool last = rr + 1 == r.rounds;
   const int n_sw = min(r.depth, r.max_iters - r.depth * rr);
   uint64_t* slot = &p.res[tol ? (rr & 1) : 0][0][0];
   const int src = rr % 3, dst = (rr + 1) % 3;
   if (n_sw >= 3 && tol && filtered_round(r, rr)) {
+    if constexpr (T == kPipeThreads) {
+      if (r.depth == kDeepTolWide && pipe_tiles(r)) {
+        do_round_pipe<T, kDeepTolWide / jac::kPipeWaves, true>(
+            rl, g.r0, g.r1, g.c0, g.c1, src, dst, &p.resd[rr & 1][0]);
+        return;
+      }
+    }
     round_tol<T, 2>(r.depth, arr(r, src), arr(r, dst), r.pitch, r.W, r.H,
                     g.r0, g.r1,
                     g.c0, g.c1, n_sw, nullptr, &p.resd[rr & 1][0]);
@@ -693,6 +768,13 @@ __device__ void run_round(const Request& r, const TileGeom& g, int rr,
     double* out = arr(r, dst);
     if constexpr (deep_for_threads(T) == kDeepWide) {
       if (n_sw > kDeep) {
+        if constexpr (T == kPipeThreads) {
+          if (!last && pipe_tiles(r)) {
+            do_round_pipe<T, kDeepWide / jac::kPipeWaves, false>(
+                rl, g.r0, g.r1, g.c0, g.c1, src, dst, nullptr);
+            return;
+          }
+        }
         if (!last)
           do_round_deep<T, kDeepWide, false, true>(in, out, r.pitch, r.W,
                                                    r.H, g.r0, g.r1, g.c0,
@@ -790,7 +872,7 @@ __global__ void __launch_bounds__(T) engine_kernel(EngineDesc E) {
     if (kind == K_INIT) {
       do_init(r, g);
     } else if (kind == K_ITER) {
-      run_round<T, NC, U>(r, g, k, p);
+      run_round<T, NC, U>(r, &s_r, g, k, p);
     } else if (kind == K_FIX && uni(s_n) < 0) {
       // round k again from its intact input, now with exact residuals (the
       // grid it writes is bit-identical to what the round wrote)
@@ -824,7 +906,7 @@ __global__ void __launch_bounds__(T) engine_kernel(EngineDesc E) {
       if (kind == K_ITER) ast(&r.pend[3 * tile + 2], (uint32_t)(k + 1));
       release_agent();
       if (kind == K_ITER) {
-        f = decide_round(p, r, k);
+        f = decide_round<T>(p, r, k);
         if (f & F_RESID) {
           ast(&p.held_tile, tile);
           release_agent();
@@ -973,9 +1055,24 @@ static double now_s() {
   return ts.tv_sec + ts.tv_nsec * 1e-9;
 }
 
+// Tile sides of engines whose rounds run as groups of waves, what a window of
+// 3, 5 or 9 columns per lane gives after sixteen sweeps (and half of the
+// first, for little work), and the time of a tile's round in us.
+constexpr int kPipeSides[] = {544, 288, 160, 96};
+constexpr double kPipeTimes[] = {300, 120, 61, 46};
+constexpr int kPipeSideN = 4;
+
+// A round of a tile of level l in us, of a problem `height` rows high (a
+// partial tile takes its share of the steps; a task costs about 8 us besides).
+static double pipe_tile_us(int height, int l) {
+  const int side = kPipeSides[l];
+  const double h = std::min(height, side);
+  return kPipeTimes[l] * (h / 2 + 38) / (side / 2 + 38) + 8;
+}
+
 // Tile side for a problem: `block` (> 0), or a rule that keeps tiles large
 // enough to amortise a task's fences and small enough to spread the problem,
-// in multiples of the deep pass's window: 112 columns at eight sweeps
+// in multiples of the window pass's window: 112 columns at eight sweeps
 // (measured on the 512-problem batch: 116-118 ms, against 158 ms with sides
 // 64/128/256/512), 96 at sixteen.
 static int pick_block(int W, int H, int block, int deep) {
@@ -985,6 +1082,59 @@ static int pick_block(int W, int H, int block, int deep) {
   if (side <= 256) return ow;
   if (side <= 1024) return 2 * ow;
   return 4 * ow;
+}
+
+// Tile sides of a batch for an engine of groups of waves (blocks[i], those
+// not given already): the largest side costs least per cell (1.0 ns a cell
+// and round at 544, 1.5 at 288, 2.5 at 160, 5.2 at 96), but a problem's
+// rounds follow each other, so the one whose rounds take longest is cut
+// finer while that is longer than the whole batch's work spread over the
+// workgroups.
+static void pick_blocks(const chm_batch_problem* probs, int n, int n_wg,
+                        std::vector<int>& blocks) {
+  struct Item {
+    double latency;
+    int i, level;
+    bool operator<(const Item& o) const { return latency < o.latency; }
+  };
+  auto rounds = [&](int i) { return (double)((probs[i].iters + 15) / 16); };
+  auto tiles = [&](int i, int side) {
+    return (double)((probs[i].width + side - 1) / side) *
+           ((probs[i].height + side - 1) / side);
+  };
+  auto tile_us = [&](int i, int l) { return pipe_tile_us(probs[i].height, l); };
+  double work = 0;  // us over all workgroups
+  std::vector<Item> heap;
+  for (int i = 0; i < n; i++) {
+    if (blocks[i] > 0) {
+      work += rounds(i) * tiles(i, blocks[i]) * 60;
+      continue;
+    }
+    int l = 0;  // no side beyond the next one that holds the problem
+    const int side = std::max(probs[i].width, probs[i].height);
+    while (l + 1 < kPipeSideN && side <= kPipeSides[l + 1]) l++;
+    blocks[i] = kPipeSides[l];
+    work += rounds(i) * tiles(i, kPipeSides[l]) * tile_us(i, l);
+    heap.push_back({rounds(i) * tile_us(i, l), i, l});
+  }
+  std::make_heap(heap.begin(), heap.end());
+  while (!heap.empty() && heap.front().latency > work / n_wg) {
+    std::pop_heap(heap.begin(), heap.end());
+    Item t = heap.back();
+    heap.pop_back();
+    if (t.level + 1 >= kPipeSideN ||
+        tiles(t.i, kPipeSides[t.level + 1]) >= (double)kMaxTiles)
+      break;  // cannot get shorter
+    const double was = rounds(t.i) * tiles(t.i, kPipeSides[t.level]) *
+                       tile_us(t.i, t.level);
+    t.level++;
+    blocks[t.i] = kPipeSides[t.level];
+    work += rounds(t.i) * tiles(t.i, kPipeSides[t.level]) *
+                tile_us(t.i, t.level) - was;
+    t.latency = rounds(t.i) * tile_us(t.i, t.level);
+    heap.push_back(t);
+    std::push_heap(heap.begin(), heap.end());
+  }
 }
 
 struct Built {
@@ -1284,6 +1434,24 @@ static void place_batch(std::vector<Built>& bl, char* arena, int n_arr) {
   }
 }
 
+// The tile side of every problem of a batch run by groups of waves: its own,
+// or pick_blocks' choice (0 for a problem that layout_batch will refuse).
+static int pipe_blocks(const chm_batch_problem* probs, int n,
+                       std::vector<int>& sides) {
+  int dev = 0, cus = 0;
+  CHM_TRY_HIP(hipGetDevice(&dev));
+  CHM_TRY_HIP(hipDeviceGetAttribute(
+      &cus, hipDeviceAttributeMultiprocessorCount, dev));
+  sides.assign(n, 0);
+  for (int i = 0; i < n; i++) {
+    const chm_batch_problem& p = probs[i];
+    if (p.width < 1 || p.height < 1 || p.iters < 1) return CHM_OK;
+    if (p.block > 0) sides[i] = p.block;
+  }
+  pick_blocks(probs, n, cus, sides);
+  return CHM_OK;
+}
+
 // One engine launch over n problems (grids seeded before the launch).
 // iters_cap > 0 caps every problem's sweeps (autotuner samples); blocks
 // (optional) overrides the tile side per problem.
@@ -1299,6 +1467,11 @@ static int batch_once(const chm_batch_problem* probs, int n,
   const int block = cfg ? cfg->block : 0;
   const int nc = cfg && cfg->panel_chunks ? cfg->panel_chunks : 1;
   const int u = cfg && cfg->rows_in_flight ? cfg->rows_in_flight : 2;
+  std::vector<int> sides;
+  if (threads == kPipeThreads && block <= 0 && !blocks) {
+    CHM_TRY(pipe_blocks(probs, n, sides));
+    blocks = sides.data();
+  }
   std::vector<Built> bl;
   size_t total = 0;
   uint64_t tiles = 0;
@@ -1558,6 +1731,28 @@ static int serve_block(int W, int H, int n_wg, int resident, int ow) {
   return 64;
 }
 
+// The same for engines of groups of waves, of their sides: a finer one where
+// it at least halves the round on this request's share of the workgroups (it
+// costs 1.5 to 2 times as much per cell, which requests that arrive beside
+// this one would miss: the burst of 24 requests of 256..8192 per side).
+static int serve_block_pipe(int W, int H, int n_wg, int resident) {
+  const int64_t share = std::max<int64_t>(1, n_wg / (1 + resident));
+  int best = kPipeSides[0];
+  double t_best = 0;
+  for (int l = 0; l < kPipeSideN; l++) {
+    const int bs = kPipeSides[l];
+    const int64_t tiles = (int64_t)((W + bs - 1) / bs) * ((H + bs - 1) / bs);
+    if (l > 0 && tiles >= (int64_t)kMaxTiles) break;
+    const double t =
+        (double)((tiles + share - 1) / share) * pipe_tile_us(H, l);
+    if (l == 0 || 2 * t <= t_best) {
+      best = bs;
+      t_best = t;
+    }
+  }
+  return best;
+}
+
 static bool pool_alloc(Server& s, size_t bytes, size_t* off) {
   for (auto it = s.free_blocks.begin(); it != s.free_blocks.end(); ++it) {
     if (it->second >= bytes) {
@@ -1750,6 +1945,8 @@ int chm_jacobi2d_batch_autotune(const chm_batch_problem* probs, int n,
   // of the deep pass's window (112 columns at eight sweeps, 96 at sixteen)
   static const int kBlocks8[] = {64, 112, 128, 224, 256, 448, 512};
   static const int kBlocks16[] = {64, 96, 128, 192, 256, 384, 512};
+  // and for groups of waves, what their windows give
+  static const int kBlocksPipe[] = {96, 160, 192, 288, 384, 512, 544};
   // size classes: one per octave of the longer side
   std::vector<int> cls(n);
   int n_cls = 0;
@@ -1763,6 +1960,8 @@ int chm_jacobi2d_batch_autotune(const chm_batch_problem* probs, int n,
   // the size rule's tiles for an engine of `threads`
   auto rule_blocks = [&](int threads) {
     std::vector<int> b(n);
+    if (threads == kPipeThreads && pipe_blocks(probs, n, b) == CHM_OK)
+      return b;
     for (int i = 0; i < n; i++)
       b[i] = pick_block(probs[i].width, probs[i].height, 0,
                         deep_for_threads(threads));
@@ -1803,7 +2002,9 @@ int chm_jacobi2d_batch_autotune(const chm_batch_problem* probs, int n,
   if (top < 0) return fail(CHM_E_DEVICE, "no autotune candidate ran");
   std::vector<int> blocks = rule_blocks(top_cfg.wg_threads);
   const bool wide = deep_for_threads(top_cfg.wg_threads) == kDeepWide;
-  const int* kBlocks = wide ? kBlocks16 : kBlocks8;
+  const int* kBlocks = top_cfg.wg_threads == kPipeThreads ? kBlocksPipe
+                       : wide                             ? kBlocks16
+                                                          : kBlocks8;
   const int n_blocks = wide ? (int)(sizeof(kBlocks16) / sizeof(int))
                             : (int)(sizeof(kBlocks8) / sizeof(int));
   // 2. tile side per size class, one class at a time (largest first)
@@ -1903,9 +2104,13 @@ int chm_jacobi2d_server_submit(void* handle, const chm_batch_problem* pb,
   const bool engine = s->mode == CHM_SERVE_ENGINE;
   int block = s->block;
   if (engine && pb->block <= 0 && block <= 0)
-    block = serve_block(pb->width, pb->height, s->e.d.n_wg,
-                        (int)s->live.size(),
-                        jac::window_out_cols(deep_tol_for_threads(s->e.threads)));
+    block = s->e.threads == kPipeThreads
+                ? serve_block_pipe(pb->width, pb->height, s->e.d.n_wg,
+                                   (int)s->live.size())
+                : serve_block(pb->width, pb->height, s->e.d.n_wg,
+                              (int)s->live.size(),
+                              jac::window_out_cols(
+                                  deep_tol_for_threads(s->e.threads)));
   const int deep = engine ? deep_for_threads(s->e.threads) : kDeep;
   CHM_TRY(check_problem(*pb, block, deep));
   Built b = build_request(*pb, block, deep);

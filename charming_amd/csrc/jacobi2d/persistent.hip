@@ -469,7 +469,6 @@ __device__ void sweepD_dispatch(int steps, const double* in, double* out,
 __device__ __noinline__ void chare_pipe(const double* in, double* out,
                                         int64_t P, int bw, int bh,
                                         RingSides rs) {
-  __shared__ PipeLds lds[CHARMING_PE_THREADS / 64 / kPipeWaves];
   PipeBlock b;
   b.in = wuni(in);
   b.out = wuni(out);
@@ -486,8 +485,7 @@ __device__ __noinline__ void chare_pipe(const double* in, double* out,
   b.lo_col = b.lo_row = 1 - kHaloRows;
   b.hi_col = b.cols.c1 - 1 + kHaloRows;
   b.hi_row = b.r1 - 1 + kHaloRows;
-  pipe_block<CHARMING_PE_THREADS, kHaloRows / kPipeWaves, false>(b, lds,
-                                                                 nullptr);
+  pipe_block<CHARMING_PE_THREADS, kHaloRows / kPipeWaves, false>(b, nullptr);
 }
 
 // The whole workgroup: the outgoing edges of the array g, D deep, into the

@@ -245,7 +245,7 @@ __device__ inline void fetch_masked(gcchar* p, int o, int lds, uint64_t m) {
       "s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\t"
       "global_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(o),
       "s"(p), "s"(lds), "s"(m)
-      : "memory", "m0");
+      : "memory");
 }
 
 // c = the K doubles at LDS byte address base + at, if row == ring_row.  In
@@ -448,7 +448,8 @@ __device__ __noinline__ void pipe_wave(int role, int lds_off) {
   auto step = [&](int u, int n) __attribute__((always_inline)) {
     const int e = (NS - u) % NS;
     __builtin_amdgcn_s_setprio(1);
-    lpair hold[2];
+    constexpr int PS = NST > 1 ? (NP + NST - 2) / (NST - 1) : NP;
+    lpair hold[PS];
     double hold_t = 0;
     shift_in(wl, er, c[e][K - 1], c[e][0]);
 #pragma unroll
@@ -524,7 +525,7 @@ __device__ __noinline__ void pipe_wave(int role, int lds_off) {
         const int orow = r0 - 2 * D + n - 1;
         const uint64_t rm = (orow >= r0 && orow < r1) ? ~0ull : 0ull;
         gdouble* rp = out + (int64_t)orow * pitch + kColOff + w0;
-        constexpr int PS = NST > 1 ? (NP + NST - 2) / (NST - 1) : NP;
+
         static_assert(NST > 1, "the shares need two sweeps per wave");
         if (s > 0) {
 #pragma unroll
@@ -621,13 +622,19 @@ struct PipeBlock {
   double ring;  // the ring's value (cols.flat)
 };
 
+// The groups' LDS, one for all passes of a kernel of T-thread workgroups.
+template <int T>
+__device__ inline PipeLds* pipe_lds() {
+  __shared__ PipeLds lds[T / 64 / kPipeWaves];
+  return lds;
+}
+
 // Workgroup-collective (T threads, all waves): 4 NST fused sweeps of the
 // block.  Groups take whole windows in turn; of an odd number the last one
 // is halved by rows (so both groups always have as many windows to do).
 // lds: one PipeLds per group of four waves.
 template <int T, int NST, bool SUM>
-__device__ __forceinline__ void pipe_block(const PipeBlock& b, PipeLds* lds,
-                                           double* sum) {
+__device__ __forceinline__ void pipe_block(const PipeBlock& b, double* sum) {
   constexpr int G = T / 64 / kPipeWaves;
   constexpr int D = kPipeWaves * NST;
   static_assert(G == 1 || G == 2, "one or two groups");
@@ -642,7 +649,7 @@ __device__ __forceinline__ void pipe_block(const PipeBlock& b, PipeLds* lds,
   const int turns = (sp.n + G - 1) / G;
   const int rows = b.r1 - b.r0;
   typedef __attribute__((address_space(3))) PipeLds lPipeLds;
-  PipeLds* my = lds + grp;
+  PipeLds* my = pipe_lds<T>() + grp;
   const int off = suni((int)(uint32_t)(uintptr_t)(lPipeLds*)my);
   for (int t = 0; t < turns; t++) {
     int win = t * G + grp, ra = b.r0, rb = b.r1;
