@@ -972,25 +972,26 @@ __global__ void init_chares_kernel(JacobiDesc d, uint64_t seed, int mode,
   const int c = blockIdx.y;
   const ChareGeom g = chare_geom(d.W, d.H, d.cr, d.cc, c);
   const int64_t P = chare_pitch(g.bw);
-  const int64_t n = (int64_t)(g.bh + 2 * kHaloRows) * P;
   double* a = d.arena + (int64_t)(2 * c) * d.chare_elems;
   double* b = a + d.chare_elems;
   const double ring = (mode == CHM_INIT_REFERENCE) ? 10.0 : boundary;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t i = e / P - (kHaloRows - 1), j = e % P - kColOff;
-    const int64_t gi = g.row0 + i, gj = g.col0 + j;
-    double v = 0.0;
-    if (j >= 1 - kHaloRows && j <= g.bw + kHaloRows && gi >= 0 &&
-        gi <= d.H + 1 && gj >= 0 && gj <= d.W + 1) {
-      const bool interior = gi >= 1 && gi <= d.H && gj >= 1 && gj <= d.W;
-      if (!interior)
-        v = ring;
-      else
-        v = (mode == CHM_INIT_REFERENCE) ? 0.0 : cell_u01(seed, gi, gj);
+  // (a row per workgroup at a time: no 64-bit division per cell)
+  for (int row = blockIdx.x; row < g.bh + 2 * kHaloRows; row += gridDim.x) {
+    const int64_t i = row - (kHaloRows - 1), gi = g.row0 + i;
+    for (int64_t e = threadIdx.x; e < P; e += blockDim.x) {
+      const int64_t j = e - kColOff, gj = g.col0 + j;
+      double v = 0.0;
+      if (j >= 1 - kHaloRows && j <= g.bw + kHaloRows && gi >= 0 &&
+          gi <= d.H + 1 && gj >= 0 && gj <= d.W + 1) {
+        const bool interior = gi >= 1 && gi <= d.H && gj >= 1 && gj <= d.W;
+        if (!interior)
+          v = ring;
+        else
+          v = (mode == CHM_INIT_REFERENCE) ? 0.0 : cell_u01(seed, gi, gj);
+      }
+      a[row * P + e] = v;
+      b[row * P + e] = v;
     }
-    a[e] = v;
-    b[e] = v;
   }
 }
 
@@ -1005,15 +1006,9 @@ __global__ void hash_chares_kernel(JacobiDesc d, int parity, int r0, int r1,
   const int lr0 = max(r0, g.row0 + 1), lr1 = min(r1, g.row0 + 1 + g.bh);
   const int lc0 = max(c0, g.col0 + 1), lc1 = min(c1, g.col0 + 1 + g.bw);
   uint64_t h = 0;
-  if (lr0 < lr1 && lc0 < lc1) {
-    const int64_t cols = lc1 - lc0, n = (int64_t)(lr1 - lr0) * cols;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
-         e += (int64_t)gridDim.x * blockDim.x) {
-      const int64_t gi = lr0 + e / cols, gj = lc0 + e % cols;
-      const int64_t li = gi - g.row0, lj = gj - g.col0;
-      h += hash_cell(gi, gj, a[li * P + kColOff + lj]);
-    }
-  }
+  for (int gi = lr0 + blockIdx.x; gi < lr1; gi += gridDim.x)
+    for (int gj = lc0 + threadIdx.x; gj < lc1; gj += blockDim.x)
+      h += hash_cell(gi, gj, a[(gi - g.row0) * P + kColOff + gj - g.col0]);
   for (int off = 32; off >= 1; off >>= 1) h += __shfl_down(h, off, 64);
   if (__lane_id() == 0 && h)
     __hip_atomic_fetch_add(out, h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

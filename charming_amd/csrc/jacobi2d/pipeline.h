@@ -448,7 +448,8 @@ __device__ __noinline__ void pipe_wave(int role, int lds_off) {
   auto step = [&](int u, int n) __attribute__((always_inline)) {
     const int e = (NS - u) % NS;
     __builtin_amdgcn_s_setprio(1);
-    constexpr int PS = NST > 1 ? (NP + NST - 2) / (NST - 1) : NP;
+    // pieces of a row in a share
+    constexpr int NSH = NST > 1 ? NST - 1 : 1, PS = (NP + NSH - 1) / NSH;
     lpair hold[PS];
     double hold_t = 0;
     shift_in(wl, er, c[e][K - 1], c[e][0]);
@@ -526,23 +527,27 @@ __device__ __noinline__ void pipe_wave(int role, int lds_off) {
         const uint64_t rm = (orow >= r0 && orow < r1) ? ~0ull : 0ull;
         gdouble* rp = out + (int64_t)orow * pitch + kColOff + w0;
 
-        static_assert(NST > 1, "the shares need two sweeps per wave");
-        if (s > 0) {
+        auto put = [&](int from) __attribute__((always_inline)) {
 #pragma unroll
           for (int x = 0; x < PS; x++) {
-            const int m = (s - 1) * PS + x;
+            const int m = from + x;
             if (m < NP)
               store_masked(rp, 16 * lane + 1024 * m, hold[x], stm[m] & rm);
           }
-          if (s == NST - 1) store_masked(rp, 8 * tail, hold_t, tail_m & rm);
-        }
-        if (s < NST - 1) {
+        };
+        if (s > 0) put((s - 1) * PS);
+        if (s > 0 && s == NST - 1) store_masked(rp, 8 * tail, hold_t, tail_m & rm);
+        if (s < NST - 1 || NST == 1) {
 #pragma unroll
           for (int x = 0; x < PS; x++) {
             const int m = s * PS + x;
             if (m < NP) hold[x] = *(const llpair*)(row_r + 128 * m);
           }
-          if (s == NST - 2) hold_t = row[tail];
+          if (s == NST - 2 || NST == 1) hold_t = row[tail];
+        }
+        if (NST == 1) {  // (nothing to overlap with: read, then store)
+          put(0);
+          store_masked(rp, 8 * tail, hold_t, tail_m & rm);
         }
         __builtin_amdgcn_sched_barrier(0);
       }

@@ -11,8 +11,10 @@
 
 #include <algorithm>
 #include <mutex>
+#include <vector>
 
 #include "jacobi2d_internal.h"
+#include "pipeline.h"
 
 namespace chm {
 namespace jac {
@@ -26,23 +28,23 @@ namespace jac {
 __global__ void init_global_kernel(double* a, double* b, int W, int H,
                                    int64_t P, uint64_t seed, int mode,
                                    double boundary) {
-  const int64_t n = (int64_t)(H + 2) * P;
   const double ring = (mode == CHM_INIT_REFERENCE) ? 10.0 : boundary;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t i = e / P;
-    const int64_t j = e % P - kColOff;
-    double v = 0.0;
-    if (j >= 0 && j <= W + 1) {
-      const bool interior = i >= 1 && i <= H && j >= 1 && j <= W;
-      if (!interior)
-        v = ring;
-      else
-        v = (mode == CHM_INIT_REFERENCE) ? 0.0 : cell_u01(seed, i, j);
+  // (a row per workgroup at a time: an index per cell costs two 64-bit
+  // divisions, which took longer than the stores)
+  for (int i = blockIdx.x; i < H + 2; i += gridDim.x)
+    for (int64_t e = threadIdx.x; e < P; e += blockDim.x) {
+      const int64_t j = e - kColOff;
+      double v = 0.0;
+      if (j >= 0 && j <= W + 1) {
+        const bool interior = i >= 1 && i <= H && j >= 1 && j <= W;
+        if (!interior)
+          v = ring;
+        else
+          v = (mode == CHM_INIT_REFERENCE) ? 0.0 : cell_u01(seed, i, j);
+      }
+      a[i * P + e] = v;
+      if (b) b[i * P + e] = v;
     }
-    a[e] = v;
-    if (b) b[e] = v;
-  }
 }
 
 // Maps a hardware workgroup id to a logical tile so that consecutive logical
@@ -55,39 +57,78 @@ __device__ inline int xcd_logical_block(int n) {
   return (i % 8) * per + i / 8;
 }
 
+// Workgroup-collective: the sum of every thread's v, in thread 0.
+__device__ inline uint64_t block_sum(uint64_t v) {
+  __shared__ uint64_t part[16];
+  for (int off = 32; off >= 1; off >>= 1) v += __shfl_down(v, off, 64);
+  if (__lane_id() == 0) part[threadIdx.x / 64] = v;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int w = 1; w < (int)(blockDim.x / 64); w++) v += part[w];
+  return v;
+}
+
+// Workgroup-collective: the exact sum of every thread's acc is added to out.
+__device__ inline void block_add_u128(uint64_t* out, u128acc acc) {
+  __shared__ u128acc part[16];
+  acc = wave_reduce_u128(acc);
+  if (__lane_id() == 0) part[threadIdx.x / 64] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < (int)(blockDim.x / 64); w++) acc_add(acc, part[w]);
+    if (acc.lo | acc.hi) atomic_add_u128(out, acc);
+  }
+}
+
+// (RES: the sweep's exact residual is added to res)
+template <int NC, int U, bool RES = false>
+__device__ __forceinline__ void plain_step(const double* __restrict__ in,
+                                           double* __restrict__ out, int W,
+                                           int H, int64_t P, int band_rows,
+                                           int n_panels, int n_tiles,
+                                           int n_blocks, uint64_t* res) {
+  const int lb = xcd_logical_block(n_blocks);
+  if (lb >= n_blocks) return;
+  const int waves = blockDim.x / 64;
+  const int tile = lb * waves + (int)(threadIdx.x / 64);
+  u128acc acc = {0, 0};
+  if (tile < n_tiles) {
+    const int panel = tile % n_panels;
+    const int band = tile / n_panels;
+    const int c0 = 1 + panel * 128 * NC;
+    const int r0 = 1 + band * band_rows;
+    const int r1 = min(r0 + band_rows, H + 1);
+    EdgeOut eo = {nullptr, nullptr, nullptr, nullptr};
+    sweep_panel<NC, U, RES, false>(in, out, P, W, H, c0, r0, r1, acc, eo);
+  }
+  if (RES) block_add_u128(res, acc);
+}
 template <int NC, int U>
 __global__ void __launch_bounds__(512)
     plain_step_kernel(const double* __restrict__ in, double* __restrict__ out,
                       int W, int H, int64_t P, int band_rows, int n_panels,
                       int n_tiles, int n_blocks) {
-  const int lb = xcd_logical_block(n_blocks);
-  if (lb >= n_blocks) return;
-  const int waves = blockDim.x / 64;
-  const int tile = lb * waves + (int)(threadIdx.x / 64);
-  if (tile >= n_tiles) return;
-  const int panel = tile % n_panels;
-  const int band = tile / n_panels;
-  const int c0 = 1 + panel * 128 * NC;
-  const int r0 = 1 + band * band_rows;
-  const int r1 = min(r0 + band_rows, H + 1);
-  u128acc acc = {0, 0};
-  EdgeOut eo = {nullptr, nullptr, nullptr, nullptr};
-  sweep_panel<NC, U, false, false>(in, out, P, W, H, c0, r0, r1, acc, eo);
+  plain_step<NC, U>(in, out, W, H, P, band_rows, n_panels, n_tiles, n_blocks,
+                    nullptr);
+}
+__global__ void __launch_bounds__(512)
+    plain_step_residual_kernel(const double* __restrict__ in,
+                               double* __restrict__ out, int W, int H,
+                               int64_t P, int band_rows, int n_panels,
+                               int n_tiles, int n_blocks, uint64_t* res) {
+  plain_step<1, 2, true>(in, out, W, H, P, band_rows, n_panels, n_tiles,
+                         n_blocks, res);
 }
 
 // Order-independent hash over interior rows [r0,r1) x cols [c0,c1).
 __global__ void hash_global_kernel(const double* g, int64_t P, int r0, int r1,
                                    int c0, int c1, uint64_t* out) {
-  const int64_t rows = r1 - r0, cols = c1 - c0;
-  const int64_t n = rows * cols;
   uint64_t h = 0;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t i = r0 + e / cols, j = c0 + e % cols;
-    h += hash_cell(i, j, g[i * P + kColOff + j]);
-  }
-  for (int off = 32; off >= 1; off >>= 1) h += __shfl_down(h, off, 64);
-  if (__lane_id() == 0)
+  for (int i = r0 + blockIdx.x; i < r1; i += gridDim.x)
+    for (int j = c0 + threadIdx.x; j < c1; j += blockDim.x)
+      h += hash_cell(i, j, g[i * P + kColOff + j]);
+  h = block_sum(h);
+  if (threadIdx.x == 0 && h)
     __hip_atomic_fetch_add(out, h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -95,16 +136,13 @@ __global__ void hash_global_kernel(const double* g, int64_t P, int r0, int r1,
 __global__ void residual_global_kernel(const double* a, const double* b,
                                        int W, int H, int64_t P,
                                        uint64_t* out) {
-  const int64_t n = (int64_t)W * H;
   u128acc acc = {0, 0};
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t i = 1 + e / W, j = 1 + e % W;
-    const int64_t o = i * P + kColOff + j;
-    acc_add(acc, res_term(a[o], b[o]));
-  }
-  acc = wave_reduce_u128(acc);
-  if (__lane_id() == 0) atomic_add_u128(out, acc);
+  for (int i = 1 + blockIdx.x; i <= H; i += gridDim.x)
+    for (int j = 1 + threadIdx.x; j <= W; j += blockDim.x) {
+      const int64_t o = i * P + kColOff + j;
+      acc_add(acc, res_term(a[o], b[o]));
+    }
+  block_add_u128(out, acc);
 }
 
 // Streaming copy of n16 16-byte words: the measured on-device copy rate the
@@ -174,6 +212,17 @@ struct StepLaunch {
 static int plan_step(const Handle* h, StepLaunch* L) {
   chm_jacobi_tuning t;
   default_tuning(&t);
+  // a grid that gives fewer than about four waves per CU in panels of 256
+  // columns x bands of 128 rows is cut finer, down to 128 x 8 (a band reads
+  // two rows more than it writes): 1500 x 1100 in 7 us a sweep, 59 as 54
+  // waves of 128 rows
+  if ((int64_t)h->W * h->H < (int64_t)1024 * 256 * 128) {
+    t.panel_chunks = h->W >= 2048 ? 2 : 1;
+    t.rows_in_flight = 2;
+    const int panels = (h->W + 128 * t.panel_chunks - 1) / (128 * t.panel_chunks);
+    const int64_t band = (int64_t)h->H * panels / 2048;
+    t.band_rows = (int)std::max<int64_t>(8, std::min<int64_t>(128, band / 8 * 8));
+  }
   if (h->tune.panel_chunks) t.panel_chunks = h->tune.panel_chunks;
   if (h->tune.rows_in_flight) t.rows_in_flight = h->tune.rows_in_flight;
   if (h->tune.band_rows) t.band_rows = h->tune.band_rows;
@@ -326,45 +375,155 @@ static int scratch_on_device(int dev, char** out) {
   return CHM_OK;
 }
 
-// Clears n words (a kernel rather than hipMemsetAsync, so the call can be
+// Copies the ring (rows 0 and H+1, columns 0 and W+1) of src to dst and
+// clears n words (here rather than by hipMemsetAsync, so the call can be
 // captured into a graph).
-__global__ void zero_words_kernel(uint64_t* p, int n) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
+__global__ void begin_noalloc_kernel(const double* src, double* dst, int W,
+                                     int H, int64_t P, uint64_t* words,
+                                     int n_words) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int T = gridDim.x * blockDim.x;
+  if (t < n_words) words[t] = 0;
+  for (int j = t; j < W + 2; j += T) {
+    dst[kColOff + j] = src[kColOff + j];
+    const int64_t o = (int64_t)(H + 1) * P + kColOff + j;
+    dst[o] = src[o];
+  }
+  for (int i = 1 + t; i <= H; i += T) {
+    const int64_t o = (int64_t)i * P + kColOff;
+    dst[o] = src[o];
+    dst[o + W + 1] = src[o + W + 1];
+  }
 }
 
-// Copies the ring (rows 0 and H+1, columns 0 and W+1) of src to dst.
-__global__ void copy_ring_kernel(const double* src, double* dst, int W, int H,
-                                 int64_t P) {
-  const int64_t n = 2 * (int64_t)(W + 2) + 2 * (int64_t)H;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    int64_t i, j;
-    if (e < 2 * (int64_t)(W + 2)) {
-      i = e < W + 2 ? 0 : H + 1;
-      j = e % (W + 2);
-    } else {
-      const int64_t k = e - 2 * (int64_t)(W + 2);
-      i = 1 + k / 2;
-      j = (k & 1) ? W + 1 : 0;
+// The hash of the interior of g (copied to `copy` on the way, if given) is
+// added to acc[0]; the last workgroup to finish writes acc[0..2] to out.
+// acc[3] counts workgroups.
+__global__ void end_noalloc_kernel(const double* g, double* copy, int W, int H,
+                                   int64_t P, uint64_t* acc, uint64_t* out) {
+  uint64_t h = 0;
+  for (int i = 1 + blockIdx.x; i <= H; i += gridDim.x)
+    for (int j = 1 + threadIdx.x; j <= W; j += blockDim.x) {
+      const int64_t o = i * P + kColOff + j;
+      const double v = g[o];
+      h += hash_cell(i, j, v);
+      if (copy) copy[o] = v;
     }
-    const int64_t o = i * P + kColOff + j;
-    dst[o] = src[o];
-  }
+  h = block_sum(h);
+  if (threadIdx.x != 0) return;
+  __hip_atomic_fetch_add(acc, h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0);  // the hash is in before the count
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  if (__hip_atomic_fetch_add(acc + 3, 1, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1)
+    for (int k = 0; k < 3; k++)
+      out[k] = __hip_atomic_load(acc + k, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Copies the interior (rows 1..H, columns 1..W) of src to dst.
-__global__ void copy_interior_kernel(const double* src, double* dst, int W,
-                                     int H, int64_t P) {
-  const int64_t n = (int64_t)W * H;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t o = (1 + e / W) * P + kColOff + 1 + e % W;
-    dst[o] = src[o];
-  }
+// 4 NST sweeps of a whole grid in one launch: a tile of tw x th cells per
+// workgroup (one per CU), swept by two groups of four waves (pipeline.h).
+// A launch per sweep was bound by its launch and by a few waves walking long
+// bands: 1021 x 683 x 100 took 5.28 ms, now 0.21; 2800 x 2800 x 200 16.3 ms,
+// now 1.04 (5 TB/s of the caches would allow 0.3; the tiles' margins and the
+// filling of their pipelines double the arithmetic); 64 x 64 x 10 345 us,
+// now 34, in five launches.
+constexpr int kPassThreads = 512;
+template <int NST>
+__global__ void __launch_bounds__(kPassThreads)
+    pass_kernel(const double* in, double* out, int W, int H, int64_t P, int tw,
+                int th, int n_cols, int n_tiles) {
+  const int tile = xcd_logical_block(n_tiles);
+  if (tile >= n_tiles) return;
+  PipeBlock b;
+  b.in = in;
+  b.out = out;
+  b.pitch = P;
+  b.cols.c0 = 1 + tile % n_cols * tw;
+  b.cols.c1 = min(b.cols.c0 + tw, W + 1);
+  b.cols.left = 0;
+  b.cols.right = W + 1;
+  b.cols.flat = false;  // the caller's ring
+  b.r0 = 1 + tile / n_cols * th;
+  b.r1 = min(b.r0 + th, H + 1);
+  b.top = 0;
+  b.bottom = H + 1;
+  b.lo_col = -kColOff;
+  b.hi_col = (int)P - kColOff - 1;
+  b.lo_row = 0;
+  b.hi_row = H + 1;
+  b.ring = 0.0;
+  pipe_block<kPassThreads, NST, false>(b, nullptr);
 }
 
-__global__ void copy_words_kernel(const uint64_t* src, uint64_t* dst, int n) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+struct PassPlan {
+  int tw, th, n_cols, n_tiles;
+};
+// Tiles of the widths a window of 3, 5 or 9 columns per lane gives, as high
+// as fill the CUs once or a few times over, by the time that takes: a tile's
+// two groups sweep half its rows each and 2 D + 10 more to fill and drain,
+// at 0.5, 0.65 or 1.0 us a row.
+static PassPlan plan_pass(int W, int H, int depth, int cus) {
+  static const double kStepUs[] = {0.5, 0.65, 1.0};
+  static const int kCols[] = {3, 5, 9};
+  PassPlan best = {0, 0, 0, 0};
+  double t_best = 0;
+  for (int k = 0; k < 3; k++) {
+    const int tw = 64 * kCols[k] - 2 * depth;
+    const int n_cols = (W + tw - 1) / tw;
+    for (int turns = 1; turns <= 8; turns++) {
+      const int rows = std::max(1, cus * turns / n_cols);
+      const int th = std::max(2, (H + rows - 1) / rows);
+      const int n = n_cols * ((H + th - 1) / th);
+      const double t = (double)((n + cus - 1) / cus) *
+                       ((th + 1) / 2 + 2 * depth + 10) * kStepUs[k];
+      if (best.tw == 0 || t < t_best) {
+        best = {tw, th, n_cols, n};
+        t_best = t;
+      }
+    }
+  }
+  return best;
+}
+
+static void launch_pass(int depth, const double* in, double* out, int W, int H,
+                        int64_t P, int cus, hipStream_t s) {
+  const PassPlan p = plan_pass(W, H, depth, cus);
+  const dim3 g((p.n_tiles + 7) / 8 * 8), b(kPassThreads);
+#define CHM_PASS(N_)                                                        \
+  case 4 * N_:                                                              \
+    pass_kernel<N_><<<g, b, 0, s>>>(in, out, W, H, P, p.tw, p.th, p.n_cols, \
+                                    p.n_tiles);                             \
+    break;
+  switch (depth) { CHM_PASS(1) CHM_PASS(2) CHM_PASS(3) CHM_PASS(4) }
+#undef CHM_PASS
+}
+
+// Sweeps per launch of `iters` sweeps whose last one is a launch of its own
+// (it leaves u_{iters-1} for the residual): sixteen, then what is left in
+// fours, then single sweeps.  An even number of launches ends in the array
+// it began in, so of an odd one a pass is split, which costs less than the
+// copy back.  Grids lower than sixteen rows are swept one at a time (a pass
+// needs the ring's rows that far apart).
+static std::vector<int> noalloc_launches(int H, int iters) {
+  std::vector<int> l;
+  int left = iters - 1;
+  while (H >= 16 && left >= 4) {
+    l.push_back(std::min(16, left / 4 * 4));
+    left -= l.back();
+  }
+  const size_t passes = l.size();
+  for (; left > 0; left--) l.push_back(1);
+  l.push_back(1);
+  if (l.size() % 2 && passes > 0 && l[passes - 1] > 4) {
+    l[passes - 1] -= 4;
+    l.insert(l.begin() + passes, 4);
+  } else if (l.size() % 2 && passes > 0 && l[0] > 4) {
+    l[0] -= 4;
+    l.insert(l.begin() + 1, 4);
+  }
+  return l;
 }
 
 static int solve_noalloc(double* grid, int W, int H, int iters,
@@ -382,8 +541,10 @@ static int solve_noalloc(double* grid, int W, int H, int iters,
                 "a %dx%d grid needs %zu bytes of scratch; the no-alloc solve "
                 "holds at most %zu",
                 W, H, bytes, kNoAllocScratchBytes - kNoAllocAccBytes);
-  int dev = 0;
+  int dev = 0, cus = 0;
   CHM_TRY_HIP(hipGetDevice(&dev));
+  CHM_TRY_HIP(hipDeviceGetAttribute(
+      &cus, hipDeviceAttributeMultiprocessorCount, dev));
   char* base = nullptr;
   CHM_TRY(scratch_on_device(dev, &base));
   uint64_t* acc = (uint64_t*)base;
@@ -392,23 +553,33 @@ static int solve_noalloc(double* grid, int W, int H, int iters,
   memset(&tmp, 0, sizeof(tmp));
   tmp.W = W;
   tmp.H = H;
-  StepLaunch L;
+  StepLaunch L, R;
   CHM_TRY(plan_step(&tmp, &L));
-  copy_ring_kernel<<<64, 256, 0, stream>>>(grid, other, W, H, P);
+  tmp.tune.panel_chunks = 1;  // the residual's one shape
+  tmp.tune.rows_in_flight = 2;
+  CHM_TRY(plan_step(&tmp, &R));
+  const int ring_blocks = std::min(64, (std::max(W, H) + 255) / 256);
+  begin_noalloc_kernel<<<ring_blocks, 256, 0, stream>>>(grid, other, W, H, P,
+                                                        acc, 4);
   double* g[2] = {grid, other};
-  for (int it = 0; it < iters; it++)
-    hipLaunchKernelGGL(L.fn, L.grid, L.block, 0, stream, g[it & 1],
-                       g[(it + 1) & 1], W, H, P, L.band_rows, L.n_panels,
-                       L.n_tiles, L.n_blocks);
-  const int cur = iters & 1;
-  zero_words_kernel<<<1, 64, 0, stream>>>(acc, 4);
-  if (iters > 0)
-    residual_global_kernel<<<1024, 256, 0, stream>>>(g[cur], g[cur ^ 1], W, H,
-                                                     P, acc + 1);
-  hash_global_kernel<<<1024, 256, 0, stream>>>(g[cur], P, 1, H + 1, 1, W + 1,
-                                               acc);
-  if (cur) copy_interior_kernel<<<1024, 256, 0, stream>>>(other, grid, W, H, P);
-  copy_words_kernel<<<1, 64, 0, stream>>>(acc, out3, 3);
+  int cur = 0;
+  if (iters > 0) {
+    const std::vector<int> launches = noalloc_launches(H, iters);
+    for (size_t i = 0; i < launches.size(); i++, cur ^= 1) {
+      if (i + 1 == launches.size())
+        plain_step_residual_kernel<<<R.grid, R.block, 0, stream>>>(
+            g[cur], g[cur ^ 1], W, H, P, R.band_rows, R.n_panels, R.n_tiles,
+            R.n_blocks, acc + 1);
+      else if (launches[i] > 1)
+        launch_pass(launches[i], g[cur], g[cur ^ 1], W, H, P, cus, stream);
+      else
+        hipLaunchKernelGGL(L.fn, L.grid, L.block, 0, stream, g[cur],
+                           g[cur ^ 1], W, H, P, L.band_rows, L.n_panels,
+                           L.n_tiles, L.n_blocks);
+    }
+  }
+  end_noalloc_kernel<<<std::min(1024, H), 256, 0, stream>>>(
+      g[cur], cur ? grid : nullptr, W, H, P, acc, out3);
   CHM_TRY_HIP(hipGetLastError());
   return CHM_OK;
 }

@@ -125,9 +125,9 @@ int chm_jacobi2d_destroy(void* handle);
 
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory: code under HIP graph capture, serving loops and harnesses that
- * forbid hipMalloc.  The plain per-launch solve of chm_jacobi2d_solve
- * (CHM_FORM_PLAIN: one sweep launch per iteration, the ring held fixed) on a
- * grid the caller owns:
+ * forbid hipMalloc.  The result of the plain per-launch solve of
+ * chm_jacobi2d_solve (the ring held fixed), with up to sixteen sweeps a
+ * launch, on a grid the caller owns:
  *   grid   device memory, 128-byte aligned, in the library's layout:
  *          height+2 rows of pitch = ((width + 18 + 15) / 16) * 16 doubles;
  *          row i holds ring column 0, interior columns 1..width and ring

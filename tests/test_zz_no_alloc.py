@@ -87,3 +87,58 @@ def test_noalloc_refuses_grid_beyond_scratch(env):
                                       out3.data_ptr())
     assert rc == -1
     assert "no-alloc solve holds at most" in L.chm_jacobi2d_last_error().decode()
+
+
+def _stepped(u0, iters):
+    from oracle import oracle as O
+    u = u0.copy()
+    for _ in range(iters):
+        prev, u = u, O.step(u)
+    return u, prev
+
+
+@pytest.mark.parametrize("w,h,iters", [
+    # passes of 16, 12, 8 and 4 sweeps, single sweeps, odd and even launches
+    (16, 16, 17), (17, 16, 5), (40, 15, 20), (1, 16, 22), (3, 40, 36),
+    (64, 64, 10), (65, 63, 9), (100, 16, 34),
+    # windows of 160, 288 and 544 columns and what is left beside them
+    (160, 100, 18), (161, 33, 21), (290, 70, 33), (545, 40, 17), (700, 300, 30),
+    (1089, 50, 19), (2000, 16, 41), (30, 2000, 25)])
+def test_noalloc_passes_any_ring(env, w, h, iters):
+    # the ring holds any values, a different one in every cell
+    from oracle import oracle as O
+    rng = np.random.default_rng(w * 7 + h + iters)
+    u0 = rng.random((h + 2, w + 2))
+    want, prev = _stepped(u0, iters)
+    grid, got = _noalloc(env, u0, w, h, iters)
+    assert np.array_equal(grid.view(np.uint64), want.view(np.uint64))
+    d = (want - prev)[1:-1, 1:-1]
+    res = sum(int(x) for x in (d * d * 2.0**56).astype(np.uint64).ravel())
+    assert got == (O.grid_hash(want), res & (2**64 - 1), res >> 64)
+
+
+def test_noalloc_captured_and_replayed(env):
+    cam, L, torch = env
+    w, h, iters = 200, 90, 30
+    P = _pitch(w)
+    rng = np.random.default_rng(3)
+    u0 = rng.random((h + 2, w + 2))
+    buf = torch.zeros((h + 2) * P, dtype=torch.float64, device="cuda")
+    out3 = torch.zeros(3, dtype=torch.int64, device="cuda")
+    view = buf.view(h + 2, P)[:, 15:17 + w]
+    # (a first call outside the capture looks the scratch buffer up)
+    assert L.chm_jacobi2d_solve_noalloc(buf.data_ptr(), w, h, 1, None,
+                                        out3.data_ptr()) == 0
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        s = torch.cuda.current_stream().cuda_stream
+        assert L.chm_jacobi2d_solve_noalloc(buf.data_ptr(), w, h, iters, s,
+                                            out3.data_ptr()) == 0
+    u = u0
+    view.copy_(torch.from_numpy(u0))
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        u, _ = _stepped(u, iters)
+        assert np.array_equal(view.cpu().numpy(), u)
