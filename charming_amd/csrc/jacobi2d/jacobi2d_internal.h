@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
+
 #include "../common/status.h"
 #include "chm_jacobi2d.h"
 #include "stencil.h"
@@ -27,6 +29,14 @@ __host__ __device__ inline void split_extent(int len, int n, int r, int* start,
 
 struct PersistentState;  // defined by the message-driven form
 
+// Two pinned buffers through which a grid goes to the host, made at the first
+// read and kept with the problem.
+struct GridReader {
+  std::mutex mu;  // reads of one problem by several threads take turns
+  double* buf[2] = {nullptr, nullptr};
+  hipEvent_t done[2] = {nullptr, nullptr};
+};
+
 struct Handle {
   chm_jacobi_problem prob;
   int form;
@@ -43,13 +53,17 @@ struct Handle {
   int graph_iters;
   // persistent form
   PersistentState* ps;
+  GridReader* reader;
 };
+
+// Launches, on the problem's stream, what writes rows [row, row + rows) of
+// the grid, ring included, to `dst` (W + 2 cells a row).
+void persistent_gather(Handle* h, double* dst, int row, int rows);
 
 // Forms implemented in other translation units.
 int persistent_create(Handle* h);
 int persistent_reset(Handle* h);
 int persistent_solve(Handle* h, chm_jacobi_result* res);
-int persistent_read_grid(Handle* h, double* out);
 int persistent_hash_region(Handle* h, int r0, int r1, int c0, int c1,
                            uint64_t* hash);
 int persistent_phase_stats(Handle* h, double* out);

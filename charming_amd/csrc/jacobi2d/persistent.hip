@@ -1014,6 +1014,28 @@ __global__ void hash_chares_kernel(JacobiDesc d, int parity, int r0, int r1,
     __hip_atomic_fetch_add(out, h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Rows [row, row + rows) of the grid, ring included, from the chares' blocks
+// to `out` (pinned host memory: bound by the link, 256 cells of a row to a
+// workgroup are whole lines but for their ends).
+__global__ void gather_chares_kernel(JacobiDesc d, int parity, double ring,
+                                     int row, int rows, double* out) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= d.W + 2) return;
+  const int cx = max(0, min((j - 1) / (d.W / d.cc), d.cc - 1));
+  for (int k = blockIdx.y; k < rows; k += gridDim.y) {
+    const int i = row + k;
+    double v = ring;
+    if (i >= 1 && i <= d.H && j >= 1 && j <= d.W) {
+      const int c = min((i - 1) / (d.H / d.cr), d.cr - 1) * d.cc + cx;
+      const ChareGeom g = chare_geom(d.W, d.H, d.cr, d.cc, c);
+      v = d.arena[(int64_t)(2 * c + parity) * d.chare_elems +
+                  (kHaloRows - 1 + i - g.row0) * chare_pitch(g.bw) + kColOff +
+                  j - g.col0];
+    }
+    out[(int64_t)k * (d.W + 2) + j] = v;
+  }
+}
+
 struct PersistentState {
   JacobiDesc desc;
   ChareGeom max_geom;
@@ -1212,25 +1234,12 @@ int persistent_hash_region(Handle* h, int r0, int r1, int c0, int c1,
   return CHM_OK;
 }
 
-int persistent_read_grid(Handle* h, double* out) {
-  PersistentState* ps = h->ps;
-  const JacobiDesc& d = ps->desc;
-  const int64_t GP = (int64_t)h->W + 2;
+void persistent_gather(Handle* h, double* dst, int row, int rows) {
   const double ring =
       (h->prob.init_mode == CHM_INIT_REFERENCE) ? 10.0 : h->prob.boundary;
-  for (int64_t e = 0; e < GP * (h->H + 2); e++) out[e] = ring;
-  for (int c = 0; c < ps->n_chares; c++) {
-    const ChareGeom g = chare_geom(d.W, d.H, d.cr, d.cc, c);
-    const int64_t P = chare_pitch(g.bw);
-    const double* a = d.arena + (int64_t)(2 * c + h->cur) * d.chare_elems +
-                      (kHaloRows - 1) * P;
-    CHM_TRY_HIP(hipMemcpy2DAsync(
-        out + (int64_t)(g.row0 + 1) * GP + g.col0 + 1, GP * sizeof(double),
-        a + P + kColOff + 1, P * sizeof(double), (size_t)g.bw * sizeof(double),
-        (size_t)g.bh, hipMemcpyDeviceToHost, h->stream));
-  }
-  CHM_TRY_HIP(hipStreamSynchronize(h->stream));
-  return CHM_OK;
+  gather_chares_kernel<<<dim3((h->W + 2 + 255) / 256, std::min(rows, 4096)),
+                         256, 0, h->stream>>>(h->ps->desc, h->cur, ring, row,
+                                              rows, dst);
 }
 
 int persistent_chare_count(Handle* h, int* n) {
