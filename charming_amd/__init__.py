@@ -290,6 +290,12 @@ def batch_run(probs, wg_threads=0, block=0, panel_chunks=0, rows_in_flight=0,
     return _pack(res, h, r, it)
 
 
+def release_memory():
+    """Give back the device memory that batches and servers keep between
+    calls (at most an eighth of the device's)."""
+    _check(jacobi_lib().chm_jacobi2d_release_memory())
+
+
 def batch_plain(probs, use_graph=False):
     """The same problems one after another, one launch per sweep (or one
     hipGraph per problem)."""

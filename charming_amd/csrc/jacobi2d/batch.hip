@@ -26,6 +26,7 @@
 #include <thread>
 #include <vector>
 
+#include "dev_cache.h"
 #include "engine_dev.h"
 #include "jacobi2d_internal.h"
 #include "pipeline.h"
@@ -1206,7 +1207,7 @@ struct Engine {
   int threads = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  std::vector<void*> dev;
+  std::vector<jac::DevBlock> dev;
   Request* h_reqs = nullptr;     // pinned request ring (serving)
   Completion* h_dones = nullptr; // pinned completion ring
   uint64_t* h_tail = nullptr;    // pinned (serving)
@@ -1217,16 +1218,17 @@ struct Engine {
 
 template <class T>
 static int dmalloc(Engine& e, T** p, size_t bytes) {
-  void* q = nullptr;
-  if (hipMalloc(&q, bytes) != hipSuccess)
+  jac::DevBlock b;
+  if (jac::DevCache::get().take(&b, bytes) != hipSuccess)
     return fail(CHM_E_NOMEM, "engine allocation of %zu bytes", bytes);
-  e.dev.push_back(q);
-  *p = (T*)q;
+  e.dev.push_back(b);
+  *p = (T*)b.p;
   return CHM_OK;
 }
 
-static void engine_free(Engine& e) {
-  for (void* p : e.dev) (void)hipFree(p);
+// idle: the engine's work has ended without an error.
+static void engine_free(Engine& e, bool idle) {
+  for (const jac::DevBlock& b : e.dev) jac::DevCache::get().put(b, idle);
   e.dev.clear();
   if (e.h_reqs) (void)hipHostFree(e.h_reqs);
   if (e.h_dones) (void)hipHostFree(e.h_dones);
@@ -1479,11 +1481,12 @@ static int batch_once(const chm_batch_problem* probs, int n,
                        deep_for_threads(threads), bl, &total, &tiles));
   Engine e;
   int rc = engine_setup(e, threads, nc, u, (uint32_t)n, tiles, false);
-  char* arena = nullptr;
-  if (rc == CHM_OK && hipMalloc(&arena, total) != hipSuccess)
+  jac::DevBlock arena;
+  if (rc == CHM_OK &&
+      jac::DevCache::get().take(&arena, total) != hipSuccess)
     rc = fail(CHM_E_NOMEM, "batch grids: %zu bytes", total);
   if (rc == CHM_OK) {
-    place_batch(bl, arena, 3);
+    place_batch(bl, (char*)arena.p, 3);
     std::vector<Request> reqs(n);
     for (int i = 0; i < n; i++) {
       init_problem<<<512, 256, 0, e.stream>>>(bl[i].r);
@@ -1533,8 +1536,8 @@ static int batch_once(const chm_batch_problem* probs, int n,
       out.res->wg_threads = threads;
     }
   }
-  if (arena) (void)hipFree(arena);
-  engine_free(e);
+  jac::DevCache::get().put(arena, rc == CHM_OK);
+  engine_free(e, rc == CHM_OK);
   return rc;
 }
 
@@ -1689,7 +1692,8 @@ static int capture_plain(PlainCtx& c, const Request& r, hipGraphExec_t* ge) {
 struct Server {
   int mode = CHM_SERVE_ENGINE;
   Engine e;
-  char* pool = nullptr;
+  jac::DevBlock mem;
+  char* pool = nullptr;  // mem's start
   size_t pool_size = 0;
   std::map<size_t, size_t> free_blocks;  // offset -> size
   std::vector<uint32_t> free_slots;
@@ -1811,7 +1815,7 @@ static void plain_worker(Server* s, int dev) {
   }
 }
 
-static void server_free(Server* s) {
+static void server_free(Server* s, bool idle) {
   if (s->worker.joinable()) {
     {
       std::lock_guard<std::mutex> lk(s->mu);
@@ -1821,9 +1825,9 @@ static void server_free(Server* s) {
     s->worker.join();
   }
   plain_ctx_free(s->pc);
-  if (s->pool) (void)hipFree(s->pool);
-  s->pool = nullptr;
-  engine_free(s->e);
+  idle = idle && s->worker_rc == CHM_OK;
+  jac::DevCache::get().put(s->mem, idle);
+  engine_free(s->e, idle);
   (void)hipDeviceSynchronize();
   delete s;
 }
@@ -1835,6 +1839,11 @@ using namespace chm;
 using namespace chm::eng;
 
 extern "C" {
+
+int chm_jacobi2d_release_memory(void) {
+  (void)jac::DevCache::get().release();
+  return CHM_OK;
+}
 
 int chm_jacobi2d_batch_run(const chm_batch_problem* probs, int n,
                            const chm_batch_config* cfg, chm_batch_result* res,
@@ -1860,13 +1869,14 @@ int chm_jacobi2d_batch_plain(const chm_batch_problem* probs, int n,
                        &tiles));
   PlainCtx c;
   int rc = plain_ctx_init(c);
-  char* arena = nullptr;
+  jac::DevBlock arena;
   std::vector<hipGraphExec_t> graphs;
   hipEvent_t e0 = nullptr, e1 = nullptr;
-  if (rc == CHM_OK && hipMalloc(&arena, total) != hipSuccess)
+  if (rc == CHM_OK &&
+      jac::DevCache::get().take(&arena, total) != hipSuccess)
     rc = fail(CHM_E_NOMEM, "batch grids: %zu bytes", total);
   if (rc == CHM_OK) {
-    place_batch(bl, arena, 2);
+    place_batch(bl, (char*)arena.p, 2);
     for (int i = 0; i < n; i++) init_problem<<<512, 256, 0, c.s>>>(bl[i].r);
     if (hipStreamSynchronize(c.s) != hipSuccess)
       rc = fail(CHM_E_HIP, "seeding the batch failed");
@@ -1925,7 +1935,7 @@ int chm_jacobi2d_batch_plain(const chm_batch_problem* probs, int n,
   for (auto ge : graphs) (void)hipGraphExecDestroy(ge);
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
-  if (arena) (void)hipFree(arena);
+  jac::DevCache::get().put(arena, rc == CHM_OK);
   plain_ctx_free(c);
   return rc;
 }
@@ -2065,7 +2075,8 @@ int chm_jacobi2d_server_start(const chm_server_config* cfg, void** handle) {
     rc = plain_ctx_init(s->pc);
   }
   // the budget is reserved up front: admission never allocates
-  if (rc == CHM_OK && hipMalloc(&s->pool, budget) != hipSuccess) {
+  if (rc == CHM_OK &&
+      jac::DevCache::get().take(&s->mem, budget) != hipSuccess) {
     (void)hipGetLastError();
     size_t fr = 0, tot = 0;
     (void)hipMemGetInfo(&fr, &tot);
@@ -2073,6 +2084,7 @@ int chm_jacobi2d_server_start(const chm_server_config* cfg, void** handle) {
               budget, fr, tot);
   }
   if (rc == CHM_OK) {
+    s->pool = (char*)s->mem.p;
     s->pool_size = budget;
     s->free_blocks[0] = budget;
     for (int i = (int)kMaxSlots - 1; i >= 0; i--) s->free_slots.push_back(i);
@@ -2090,7 +2102,7 @@ int chm_jacobi2d_server_start(const chm_server_config* cfg, void** handle) {
       __atomic_store_n(s->e.h_stop, 2u, __ATOMIC_SEQ_CST);
       (void)engine_wait(s->e, 60, nullptr);
     }
-    server_free(s);
+    server_free(s, false);
     return keep;
   }
   *handle = s;
@@ -2239,7 +2251,7 @@ int chm_jacobi2d_server_stop(void* handle, int abort_now, double timeout_s) {
     const int rc2 = engine_wait(s->e, 60.0, nullptr);
     if (rc == CHM_OK) rc = rc2;
   }
-  server_free(s);
+  server_free(s, rc == CHM_OK);
   return rc;
 }
 

@@ -1,0 +1,133 @@
+// Device memory of the batched and served forms, kept between calls: grids
+// and queues are gigabytes that a call needs for tens of milliseconds, and
+// taking 16 GiB from the driver and giving it back costs 240-480 ms (a served
+// burst of 24 requests, 16 GiB of pool: 470 ms, now 134; 512 problems, 17 GB of
+// grids: 110-490, now 75).
+//
+// What is kept is bounded (an eighth of the device's memory, kBlocks blocks;
+// the longest unused go first), holds no data (every user writes what it
+// reads), is given back when any allocation of this library fails, when a
+// block has not been used for kKeepSeconds and another is returned, and by
+// chm_jacobi2d_release_memory().  A block is kept only once the work that used
+// it has ended, so any stream may take it next.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <algorithm>
+#include <chrono>
+#include <mutex>
+
+namespace chm {
+namespace jac {
+
+struct DevBlock {
+  void* p = nullptr;
+  size_t bytes = 0;  // may exceed what was asked for
+  int dev = 0;       // the device it is on
+};
+
+class DevCache {
+ public:
+  // (never destroyed: its blocks go with the process)
+  static DevCache& get() {
+    static DevCache* c = new DevCache;
+    return *c;
+  }
+
+  // At least `bytes` of the current device: the smallest kept block of up to
+  // a quarter and 1 MiB more, or new memory.
+  hipError_t take(DevBlock* b, size_t bytes) {
+    hipError_t e = hipGetDevice(&b->dev);
+    if (e != hipSuccess) return e;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      Kept* best = nullptr;
+      for (int i = 0; i < n_; i++)
+        if (kept_[i].b.dev == b->dev && kept_[i].b.bytes >= bytes &&
+            kept_[i].b.bytes - bytes <= bytes / 4 + (1 << 20) &&
+            (!best || kept_[i].b.bytes < best->b.bytes))
+          best = &kept_[i];
+      if (best) {
+        *b = best->b;
+        *best = kept_[--n_];
+        return hipSuccess;
+      }
+    }
+    b->bytes = bytes;
+    return alloc(&b->p, bytes);
+  }
+
+  // hipMalloc, with what is kept given back if it fails.
+  template <class T>
+  hipError_t alloc(T** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess || !release()) return e;
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
+  }
+
+  // Returns a block; `idle` says that nothing uses it any more.
+  void put(DevBlock b, bool idle) {
+    if (!b.p) return;
+    size_t total = 0;
+    if (!idle || hipDeviceTotalMem(&total, b.dev) != hipSuccess ||
+        b.bytes > total / 8) {
+      (void)hipFree(b.p);
+      return;
+    }
+    const auto now = Clock::now();
+    void* out[kBlocks + 1];
+    int n_out = 0;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      for (;;) {
+        size_t sum = b.bytes;
+        int old = -1;
+        for (int i = 0; i < n_; i++) {
+          if (kept_[i].b.dev != b.dev) continue;
+          sum += kept_[i].b.bytes;
+          if (old < 0 || kept_[i].t < kept_[old].t) old = i;
+        }
+        if (old < 0 || (sum <= total / 8 && n_ < kBlocks &&
+                        now - kept_[old].t < std::chrono::seconds(kKeepSeconds)))
+          break;
+        out[n_out++] = kept_[old].b.p;
+        kept_[old] = kept_[--n_];
+      }
+      if (n_ < kBlocks)
+        kept_[n_++] = Kept{b, now};
+      else
+        out[n_out++] = b.p;
+    }
+    // (outside the lock: a free may wait for work on the device)
+    for (int i = 0; i < n_out; i++) (void)hipFree(out[i]);
+  }
+
+  // Gives everything back; false if nothing was kept.
+  bool release() {
+    void* out[kBlocks];
+    int n_out = 0;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      while (n_ > 0) out[n_out++] = kept_[--n_].b.p;
+    }
+    for (int i = 0; i < n_out; i++) (void)hipFree(out[i]);
+    return n_out > 0;
+  }
+
+ private:
+  using Clock = std::chrono::steady_clock;
+  static constexpr int kBlocks = 48;
+  static constexpr int kKeepSeconds = 10;
+  struct Kept {
+    DevBlock b;
+    Clock::time_point t;
+  };
+  std::mutex mu_;
+  Kept kept_[kBlocks];
+  int n_ = 0;
+};
+
+}  // namespace jac
+}  // namespace chm

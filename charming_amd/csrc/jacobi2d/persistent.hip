@@ -42,6 +42,7 @@ __device__ void jacobi_work(void* token);
 #include <algorithm>
 #include <vector>
 
+#include "dev_cache.h"
 #include "jacobi2d_internal.h"
 #include "pipeline.h"
 
@@ -1081,7 +1082,9 @@ int persistent_create(Handle* h) {
     // watchdog: generous for the largest grids this form is used on
     // (16384^2 x 1000 sweeps takes about a second)
     cfg.timeout_s = 120.0;
-    const int rc = chm_init(0, nullptr, &cfg);
+    int rc = chm_init(0, nullptr, &cfg);
+    if (rc == CHM_E_NOMEM && DevCache::get().release())
+      rc = chm_init(0, nullptr, &cfg);
     if (rc != CHM_OK) return fail(rc, "chm_init: %s", chm_last_error());
   }
   g_runtime_users++;
@@ -1122,13 +1125,13 @@ int persistent_create(Handle* h) {
       (size_t)ps->n_chares * 2 * (size_t)d.chare_elems * sizeof(double);
   const size_t stage_bytes = (size_t)ps->n_chares * N_NEIGHBORS *
                              (size_t)d.stage_elems * sizeof(double);
-  if (hipMalloc(&d.arena, arena_bytes) != hipSuccess ||
-      hipMalloc(&d.staging, stage_bytes) != hipSuccess ||
-      hipMalloc(&d.res_acc, 4 * sizeof(uint64_t)) != hipSuccess ||
-      hipMalloc(&d.phase, (size_t)ps->n_chares * 4 * sizeof(uint64_t)) !=
-          hipSuccess ||
-      hipMalloc(&d.recv_ticks, (size_t)ps->n_chares * sizeof(uint64_t)) !=
-          hipSuccess)
+  auto alloc = [](auto** p, size_t bytes) {
+    return DevCache::get().alloc(p, bytes) == hipSuccess;
+  };
+  if (!alloc(&d.arena, arena_bytes) || !alloc(&d.staging, stage_bytes) ||
+      !alloc(&d.res_acc, 4 * sizeof(uint64_t)) ||
+      !alloc(&d.phase, (size_t)ps->n_chares * 4 * sizeof(uint64_t)) ||
+      !alloc(&d.recv_ticks, (size_t)ps->n_chares * sizeof(uint64_t)))
     return fail(CHM_E_NOMEM, "persistent form allocation (%zu + %zu bytes)",
                 arena_bytes, stage_bytes);
   return persistent_reset(h);

@@ -14,6 +14,7 @@
 #include <new>
 #include <vector>
 
+#include "dev_cache.h"
 #include "jacobi2d_internal.h"
 #include "pipeline.h"
 
@@ -683,7 +684,8 @@ int chm_jacobi2d_create(const chm_jacobi_problem* prob, int form,
       rc = fail(CHM_E_NOMEM, "host alloc");
       break;
     }
-    if (hipMalloc(&h->d_acc, 4 * sizeof(uint64_t)) != hipSuccess) {
+    if (DevCache::get().alloc(&h->d_acc, 4 * sizeof(uint64_t)) !=
+        hipSuccess) {
       rc = fail(CHM_E_NOMEM, "scratch alloc");
       break;
     }
@@ -692,8 +694,8 @@ int chm_jacobi2d_create(const chm_jacobi_problem* prob, int form,
       break;
     }
     const size_t bytes = array_elems(h->W, h->H) * sizeof(double);
-    if (hipMalloc(&h->grid[0], bytes) != hipSuccess ||
-        hipMalloc(&h->grid[1], bytes) != hipSuccess) {
+    if (DevCache::get().alloc(&h->grid[0], bytes) != hipSuccess ||
+        DevCache::get().alloc(&h->grid[1], bytes) != hipSuccess) {
       rc = fail(CHM_E_NOMEM, "grid alloc of 2 x %zu bytes", bytes);
       break;
     }
@@ -820,8 +822,8 @@ int chm_hbm_copy_probe(size_t bytes, int reps, double* ms_per_copy) {
   CHM_TRY_HIP(hipEventCreate(&e0));
   CHM_TRY_HIP(hipEventCreate(&e1));
   int rc = CHM_OK;
-  if (hipMalloc(&a, n16 * 16) != hipSuccess ||
-      hipMalloc(&b, n16 * 16) != hipSuccess) {
+  if (DevCache::get().alloc(&a, n16 * 16) != hipSuccess ||
+      DevCache::get().alloc(&b, n16 * 16) != hipSuccess) {
     rc = fail(CHM_E_NOMEM, "copy probe alloc");
   } else {
     (void)hipMemsetAsync(a, 0, n16 * 16, s);

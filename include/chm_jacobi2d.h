@@ -215,6 +215,11 @@ int chm_jacobi2d_batch_run(const chm_batch_problem* probs, int n,
                            uint64_t* hashes, uint64_t* residuals,
                            int* iters_done);
 
+/* Batches and servers keep the device memory they took for the next one, up
+ * to an eighth of the device's; it goes back when an allocation of this
+ * library fails, or here. */
+int chm_jacobi2d_release_memory(void);
+
 /* The same problems solved one after another in the plain per-iteration
  * form (use_graph = 0: one launch per sweep; 1: each problem's sweeps
  * captured beforehand as a hipGraph and replayed).  Same outputs. */
