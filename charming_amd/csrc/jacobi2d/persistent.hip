@@ -119,7 +119,7 @@ struct Block : charm::chare {
   int neighbor_index[N_NEIGHBORS];
   int neighbor_count;
   int recv_count;
-  int end_count;
+  int end_count;  // (from 0 at creation: a child may report before init)
   int block_width, block_height;
   int64_t pitch;
   int n_iters, iter;
@@ -131,7 +131,7 @@ struct Block : charm::chare {
   // times the same way): device wall-clock ticks
   uint64_t t_sweep, t_send, t_wait, t_mark;
 
-  __device__ Block() {}
+  __device__ Block() : end_count(0) {}
   __device__ void init(void* arg);
   __device__ size_t halo_bytes(int k) const;
   __device__ void fill_corners(double* const* bufs);
@@ -139,6 +139,7 @@ struct Block : charm::chare {
   __device__ void put_edges(const double* g, int D, int parity);
   __device__ void recv_ghosts(void* arg);
   __device__ void update();
+  __device__ void finish();
   __device__ void end(void* arg);
 };
 
@@ -583,7 +584,6 @@ __device__ void Block::init(void* arg) {
     for (int k = 0; k < N_NEIGHBORS; k++)
       neighbor_count += (neighbor_index[k] >= 0);
     recv_count = 0;
-    end_count = 0;
     t_sweep = t_send = t_wait = 0;
     grids[0] = d.arena + (int64_t)(2 * index) * d.chare_elems +
                (kHaloRows - 1) * pitch;
@@ -628,7 +628,7 @@ __device__ size_t Block::halo_bytes(int k) const {
   return sizeof(double) + sizeof(double) * len;
 }
 
-// Thread 0: with halos D >= 2 deep the four (D-1) x (D-1) corner blocks go
+// The workgroup: with halos D >= 2 deep the four (D-1) x (D-1) corner blocks go
 // to the diagonal neighbours, taken from the top and bottom edges already
 // written (a diagonal neighbour implies both): the block nearest each
 // corner of the chare, rows in order.  bufs[k] = [dir slot | payload].
@@ -640,24 +640,24 @@ __device__ void Block::fill_corners(double* const* bufs) {
   const int bw = block_width, n = D - 1;
   const double* top = bufs[TOP] + 1;                 // rows 1 .. D
   const double* bot = bufs[BOTTOM] + 1 + (int64_t)bw;  // rows bh-D+2 .. bh
-  for (int i = 0; i < n; i++)
-    for (int j = 0; j < n; j++) {
-      if (neighbor_index[TOP_LEFT] >= 0)
-        bufs[TOP_LEFT][1 + i * n + j] = top[(int64_t)i * bw + j];
-      if (neighbor_index[TOP_RIGHT] >= 0)
-        bufs[TOP_RIGHT][1 + i * n + j] = top[(int64_t)i * bw + bw - n + j];
-      if (neighbor_index[BOTTOM_LEFT] >= 0)
-        bufs[BOTTOM_LEFT][1 + i * n + j] = bot[(int64_t)i * bw + j];
-      if (neighbor_index[BOTTOM_RIGHT] >= 0)
-        bufs[BOTTOM_RIGHT][1 + i * n + j] = bot[(int64_t)i * bw + bw - n + j];
-    }
+  for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
+    const int i = e / n, j = e % n;
+    if (neighbor_index[TOP_LEFT] >= 0)
+      bufs[TOP_LEFT][1 + i * n + j] = top[(int64_t)i * bw + j];
+    if (neighbor_index[TOP_RIGHT] >= 0)
+      bufs[TOP_RIGHT][1 + i * n + j] = top[(int64_t)i * bw + bw - n + j];
+    if (neighbor_index[BOTTOM_LEFT] >= 0)
+      bufs[BOTTOM_LEFT][1 + i * n + j] = bot[(int64_t)i * bw + j];
+    if (neighbor_index[BOTTOM_RIGHT] >= 0)
+      bufs[BOTTOM_RIGHT][1 + i * n + j] = bot[(int64_t)i * bw + bw - n + j];
+  }
 }
 
 __device__ void Block::send_boundaries() {
   // (jacobi2d.cu:152-194) sends tagged with the iteration: four edges
   // `depth` deep, and with deeper halos the four corner blocks, copied
   // from the staging buffers
-  if (threadIdx.x == 0) fill_corners(boundaries);
+  fill_corners(boundaries);
   __syncthreads();
   for (int k = 0; k < N_NEIGHBORS; k++) {
     if (neighbor_index[k] < 0) continue;
@@ -852,17 +852,16 @@ __device__ void Block::update() {
     __shared__ double* s_dst[N_NEIGHBORS];
     for (int k = 0; k < N_NEIGHBORS; k++) {
       double* d = (neighbor_index[k] >= 0) ? boundaries[k] : nullptr;
-      if (zc && neighbor_index[k] >= 0) {
+      if (zc && !put && neighbor_index[k] >= 0) {
         charm::message m;
         d = (double*)block_proxy->alloc(m, neighbor_index[k], 1,
-                                        put ? sizeof(double) : halo_bytes(k),
-                                        iter + steps);
+                                        halo_bytes(k), iter + steps);
         if (threadIdx.x == 0) {
           s_env[k] = m.env;
           s_off[k] = m.offset;
           if (d) {
             ((int*)d)[0] = opposite_side(k);
-            ((int*)d)[1] = put ? 1 : 0;
+            ((int*)d)[1] = 0;
           }
         }
       }
@@ -911,8 +910,16 @@ __device__ void Block::update() {
     }
     __syncthreads();
     // the halos of u_{iter} leave before the interior is swept
-    if (!done && zc) {
-      if (threadIdx.x == 0 && !put) fill_corners(s_dst);
+    if (!done && put) {
+      // one lane per neighbour: the slot word, "placed"
+      const int k = threadIdx.x;
+      const int to = k < N_NEIGHBORS ? neighbor_index[k] : -1;
+      charm::rt::send_words(
+          block_proxy->id, 1, iter, N_NEIGHBORS,
+          to >= 0 ? block_proxy->pe_of(to) : 0, to,
+          (uint64_t)(uint32_t)opposite_side(k & 7) | (1ull << 32));
+    } else if (!done && zc) {
+      fill_corners(s_dst);
       for (int k = 0; k < N_NEIGHBORS; k++) {
         if (neighbor_index[k] < 0) continue;
         charm::message m;
@@ -943,18 +950,36 @@ __device__ void Block::update() {
         ph[2] = t_wait;
         ph[3] = (uint64_t)n_iters;
       }
-      block_proxy->invoke(0, 2);
+      finish();
       return;
     }
     if (neighbor_count > 0) return;
   }
 }
 
+// The end of the solve is counted up a tree of chares, kEndFan to a parent
+// (all of 256 reporting to chare 0 kept its PE busy for 0.8 ms): each sends
+// one message when it and its children are done, the root one to itself.
+constexpr int kEndFan = 4;
+
+__device__ void Block::finish() {
+  if (charm::chare::i == 0)
+    block_proxy->invoke(0, 2);
+  else
+    end(nullptr);
+}
+
 __device__ void Block::end(void* arg) {
   __shared__ int fin;
-  if (threadIdx.x == 0) fin = (++end_count == charm::chare::n);
+  const int i = charm::chare::i, n = charm::chare::n;
+  const int children = max(0, min(kEndFan, n - 1 - kEndFan * i));
+  if (threadIdx.x == 0) fin = (++end_count == children + 1);
   __syncthreads();
-  if (fin) charm::end();
+  if (!fin) return;
+  if (i == 0)
+    charm::end();
+  else
+    block_proxy->invoke((i - 1) / kEndFan, 2);
 }
 
 // ---------------------------------------------------------------------------

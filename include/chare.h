@@ -25,6 +25,8 @@ namespace rt {
 __device__ PeState* pe_state();
 __device__ void* heap_alloc(size_t bytes, size_t align);
 __device__ void raise_error(uint32_t code, uint32_t aux);
+__device__ bool send_all(int chare_id, int ep, const void* buf,
+                         uint64_t payload, int n);
 }  // namespace rt
 
 struct chare {
@@ -249,6 +251,10 @@ struct chare_proxy : chare_proxy_base {
 
   inline __device__ void invoke_all(int ep) { invoke_all(ep, nullptr, 0); }
   inline __device__ void invoke_all(int ep, void* buf, size_t size) {
+    // at most one chare a PE under the default map: chare i is on PE i
+    if (!loc_map && n_total <= n_pes() &&
+        rt::send_all(id, ep, buf, size, n_total))
+      return;
     for (int i = 0; i < n_total; i++) invoke(i, ep, buf, size);
   }
 

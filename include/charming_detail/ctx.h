@@ -118,7 +118,6 @@ struct PeState {
   UserExtent user_free[kUserExtents];
   int n_waits;         // valid entries of waits[]
   AsyncWait waits[ASYNC_WAIT_MAX];
-  uint64_t read_pos;   // logical position of the next inbox message
   uint64_t heap_used;  // bump allocator in the PE's heap slice
   uint32_t arena_used; // deferred arena bump pointer
   uint32_t seq;

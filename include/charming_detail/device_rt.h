@@ -17,8 +17,9 @@
 //   producer (thread 0): ready[dst][pos/64 mod N] = pos/64 + 1     (release;
 //                        batched: one release covers every message an
 //                        entry method sent, see flush_publish)
-//   consumer (thread 0): poll ready[me][read/64 mod N] == read/64+1 (relaxed)
-//                        then an agent-scope acquire fence
+//   consumer (wave 0):   poll ready[me][read/64 mod N] == read/64+1 (relaxed)
+//                        and the kAhead - 1 words after it, then one
+//                        agent-scope acquire fence for all that are published
 //   all threads:         run the entry method on the message in place
 //   consumer (thread 0): read += slot; head[me] = read             (relaxed,
 //                        after the reads completed)
@@ -44,6 +45,12 @@ static __constant__ Ctx g_ctx;
 
 constexpr uint64_t kFail = ~0ull;
 constexpr int kMaxPending = 16;
+// Ready words read by one poll.  A message costs its consumer a chain of loads
+// that all miss after the acquire has emptied the CU's L1, 4-5 us; those found
+// published together share one acquire and the lines it brings back.  16
+// words are one or two cache lines.
+constexpr int kAhead = 16;
+constexpr uint64_t kSmallPayload = 64;  // a lane's own copy, see send_all
 enum : int { CMD_EXIT = 0, CMD_INBOX = 1, CMD_REVIVED = 2, CMD_ASYNC = 3 };
 
 // Workgroup-shared scratch used to broadcast thread 0's decisions.  The
@@ -69,6 +76,11 @@ struct Lds {
   void* work;        // token of the program's work hook (request_work)
   int has_work;
   uint64_t t_found;  // wall clock when the current message was found
+  uint64_t read_pos;   // logical position of the next inbox message
+  uint64_t seen_base;  // granule from which `seen` counts
+  uint64_t seen;       // bit k: granule seen_base + k starts a message that
+                       // is published and acquired
+  Stats stats;         // the PE's, stored at the end of the launch
   int cmd;
   int arg;
   int n;
@@ -254,7 +266,7 @@ __device__ uint64_t reserve(int dst, uint64_t slot) {
         raise_error(ERR_SPIN_LIMIT, (uint32_t)dst);
         return kFail;
       }
-      pe_state()->stats.send_spins++;
+      lds().stats.send_spins++;
       __builtin_amdgcn_s_sleep(2);
     }
   }
@@ -272,7 +284,7 @@ __device__ void queue_publish(int dst, uint64_t pos) {
       &c.ready[(uint64_t)dst * n_granules() + (g & (n_granules() - 1))];
   L.pend_tag[L.n_pend] = g + 1;
   L.n_pend++;
-  pe_state()->stats.sent++;
+  lds().stats.sent++;
 }
 
 // Workgroup-collective: reserve a message in the destination's ring and
@@ -327,6 +339,131 @@ __device__ void send_msg(int dst, msgtype type, int chare_id, int chare_idx,
   wave_drain();
   __syncthreads();
   if (threadIdx.x == 0) queue_publish(to, pos);
+}
+
+#ifndef CHARMING_GPU_LEVEL
+// Workgroup-collective: every thread with `mine` sends one message of `bytes`
+// (at most kSmallPayload, the same for all) to entry method ep of chare idx on
+// PE dst.  Sent one after another messages cost their sender 2-8 us each;
+// here the lanes reserve, write and publish together, with one release.  A
+// lane whose destination is full goes on once there is room, with nothing
+// held back meanwhile.  Thread 0's chare_id, ep and refnum count (L.snd).
+__device__ void send_lanes(bool mine, int dst, int idx, const char* from,
+                           uint64_t bytes) {
+  const Ctx& c = g_ctx;
+  Lds& L = lds();
+  const uint64_t alloc = envelope::alloc_size(msgtype::regular, bytes);
+  const uint64_t slot = (alloc + kGranule - 1) & ~(kGranule - 1);
+  uint64_t pos = 0;
+  bool room = false;
+  auto write = [&] {
+    char* m = c.rings + (uint64_t)dst * c.ring_stride +
+              (pos & (c.ring_bytes - 1));
+    new (m) envelope(msgtype::regular, alloc);
+    m += sizeof(envelope);
+    new (m) regular_msg(L.snd.chare_id, idx, L.snd.ep, L.snd.refnum);
+    m += sizeof(regular_msg);
+    for (uint64_t k = 0; k < bytes; k++) m[k] = from[k];
+  };
+  auto publish = [&] {
+    const uint64_t g = pos / kGranule;
+    st_relaxed(&c.ready[(uint64_t)dst * n_granules() +
+                        (g & (n_granules() - 1))],
+               g + 1);
+    atomicAdd(&L.stats.sent, 1ull);
+  };
+  if (mine) {
+    pos = __hip_atomic_fetch_add(&c.tails[(uint64_t)dst * 16], slot,
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    room = pos + slot - ld_relaxed(&c.heads[(uint64_t)dst * 16]) <=
+           c.ring_bytes;
+    if (room) write();
+  }
+  wave_drain();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    release_fence();
+    flush_publish();
+  }
+  __syncthreads();
+  if (room) publish();
+  bool late = mine && !room;
+  for (uint64_t spins = 1; __any(late); spins++) {
+    if (late) {
+      if (pos + slot - ld_relaxed(&c.heads[(uint64_t)dst * 16]) <=
+          c.ring_bytes) {
+        write();
+        release_fence();
+        publish();
+        late = false;
+      } else if (dst == pe_index()) {
+        raise_error(ERR_SELF_RING_FULL, (uint32_t)slot);
+        late = false;
+      } else if (stopping()) {
+        late = false;
+      } else if (c.spin_limit && spins > c.spin_limit) {
+        raise_error(ERR_SPIN_LIMIT, (uint32_t)dst);
+        late = false;
+      } else {
+        atomicAdd(&L.stats.send_spins, 1ull);
+      }
+    }
+    __builtin_amdgcn_s_sleep(2);
+  }
+}
+#endif
+
+// Workgroup-collective: one message with thread 0's payload for entry method
+// ep of each of the n chares, chare i on PE i (n <= n_pes).  False, with
+// nothing sent, where the payload is more than a lane should copy.
+__device__ __noinline__ bool send_all(int chare_id, int ep, const void* buf,
+                                      uint64_t payload, int n) {
+#ifdef CHARMING_GPU_LEVEL
+  return false;
+#else
+  Lds& L = lds();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    L.snd.buf = buf;
+    L.snd.payload = payload;
+    L.snd.chare_id = chare_id;
+    L.snd.ep = ep;
+    L.snd.refnum = -1;
+  }
+  __syncthreads();
+  const uint64_t bytes = L.snd.payload;
+  if (bytes > kSmallPayload ||
+      envelope::alloc_size(msgtype::regular, bytes) + kGranule >
+          g_ctx.max_msg_bytes)
+    return false;
+  for (int base = 0; base < n; base += blockDim.x) {
+    const int i = base + (int)threadIdx.x;
+    send_lanes(i < n, i, i, (const char*)L.snd.buf, bytes);
+  }
+  __syncthreads();
+  return true;
+#endif
+}
+
+// Workgroup-collective: thread k < n sends its own `word` to entry method ep
+// of chare idx on PE dst (idx < 0: none), all with one reference number.
+__device__ void send_words(int chare_id, int ep, int refnum, int n, int dst,
+                           int idx, uint64_t word) {
+#ifdef CHARMING_GPU_LEVEL
+  raise_error(ERR_UNSUPPORTED, 0);
+#else
+  Lds& L = lds();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    L.snd.chare_id = chare_id;
+    L.snd.ep = ep;
+    L.snd.refnum = refnum;
+  }
+  __syncthreads();
+  send_lanes((int)threadIdx.x < n && idx >= 0, dst, idx, (const char*)&word,
+             sizeof(word));
+  __syncthreads();
+#endif
 }
 
 // ---------------------------------------------------------------------------
@@ -416,7 +553,7 @@ __device__ void defer(const char* msg, uint64_t alloc, int chare_id,
       d.seq = ps->seq++;
       ps->arena_used += need;
       ps->n_deferred++;
-      ps->stats.deferred++;
+      lds().stats.deferred++;
       L.arg = e;
       L.ptr = arena() + d.offset;
     }
@@ -442,7 +579,7 @@ __device__ __noinline__ bool dispatch(envelope* env) {
       return true;
     }
     if (threadIdx.x == 0)
-      pe_state()->stats.overhead_ticks += wall_clock64() - lds().t_found;
+      lds().stats.overhead_ticks += wall_clock64() - lds().t_found;
     const bool ok = t.proxies[id]->call(m->chare_idx, m->ep_id,
                                         (char*)m + sizeof(regular_msg),
                                         m->refnum);
@@ -471,61 +608,95 @@ __device__ inline bool wait_satisfied(const AsyncWait& w) {
   return true;
 }
 
-// Thread 0: wait for work.  Revived messages go first (in arrival order),
-// then the inbox in FIFO order, then satisfied async waits.
-__device__ int poll_next() {
+// Thread 0: the next revived message, in arrival order; -1 if there is none.
+__device__ int poll_revived() {
+  PeState* ps = pe_state();
+  Lds& L = lds();
+  if (ps->n_revived <= 0) return -1;
+  int best = -1;
+  for (int i = 0; i < ps->hw; i++)
+    if (ps->deferred[i].state == 2 &&
+        (best < 0 || ps->deferred[i].seq < ps->deferred[best].seq))
+      best = i;
+  if (best < 0) {
+    ps->n_revived = 0;
+    return -1;
+  }
+  L.t_found = wall_clock64();
+  ps->deferred[best].state = 3;  // being processed
+  ps->n_revived--;
+  L.arg = best;
+  L.ptr = arena() + ps->deferred[best].offset;
+  return CMD_REVIVED;
+}
+
+// Thread 0: a satisfied async wait or the order to stop; -1 if neither.
+__device__ int poll_rest(uint32_t spins) {
   const Ctx& c = g_ctx;
   PeState* ps = pe_state();
   Lds& L = lds();
-  const uint64_t NG = n_granules();
-  const uint64_t* rdy = c.ready + (uint64_t)pe_index() * NG;
-  char* ring = c.rings + (uint64_t)pe_index() * c.ring_stride;
-  for (uint32_t spins = 0;; spins++) {
-    if (ps->n_revived > 0) {
-      int best = -1;
-      for (int i = 0; i < ps->hw; i++)
-        if (ps->deferred[i].state == 2 &&
-            (best < 0 || ps->deferred[i].seq < ps->deferred[best].seq))
-          best = i;
-      if (best >= 0) {
-        L.t_found = wall_clock64();
-        ps->deferred[best].state = 3;  // being processed
-        ps->n_revived--;
-        L.arg = best;
-        L.ptr = arena() + ps->deferred[best].offset;
-        return CMD_REVIVED;
-      }
-      ps->n_revived = 0;
-    }
-    const uint64_t g = ps->read_pos / kGranule;
-    if (ld_relaxed(&rdy[g & (NG - 1)]) == g + 1) {
+  if (ps->n_waits > 0) {
+    for (int i = 0; i < ASYNC_WAIT_MAX; i++) {
+      AsyncWait& w = ps->waits[i];
+      if (!w.valid || !wait_satisfied(w)) continue;
       L.t_found = wall_clock64();
       fence_acquire();
-      L.ptr = ring + (ps->read_pos & (c.ring_bytes - 1));
+      w.valid = 0;
+      ps->n_waits--;
+      L.arg = w.proxy;
+      L.n = w.idx;
+      L.pos = (uint64_t)w.ep;
+      return CMD_ASYNC;
+    }
+  }
+  if (ld_relaxed(&c.ctl[CTL_TERM]) != 0) return CMD_EXIT;
+  if ((spins & 255) == 255) {
+    if (*c.host_abort) {
+      raise_error(ERR_HOST_ABORT, 0);
+      return CMD_EXIT;
+    }
+    L.stats.idle_polls++;
+  }
+  return -1;
+}
+
+// Threads 0 .. kAhead-1 of the first wave, or thread 0 alone (which then
+// reads one word a poll): wait for work.  Revived messages go first (in
+// arrival order), then the inbox in FIFO order, then satisfied async waits.
+__device__ int poll_next() {
+  const Ctx& c = g_ctx;
+  Lds& L = lds();
+  const uint32_t l = threadIdx.x;
+  const uint64_t NG = n_granules();
+  const uint64_t* rdy = c.ready + (uint64_t)pe_index() * NG;
+  const uint64_t pos = L.read_pos, g = pos / kGranule;
+  const uint64_t at = g - L.seen_base;
+  const bool known = at < kAhead && ((L.seen >> at) & 1) != 0;
+  for (uint32_t spins = 0;; spins++) {
+    int cmd = -1;
+    if (l == 0) cmd = poll_revived();
+    cmd = __builtin_amdgcn_readfirstlane(cmd);
+    if (cmd >= 0) return cmd;
+    uint64_t found = 0;
+    if (!known) {
+      found = __ballot(ld_relaxed(&rdy[(g + l) & (NG - 1)]) == g + l + 1);
+      if (found & 1) fence_acquire();
+    }
+    if (known || (found & 1)) {
+      if (l == 0) {
+        L.t_found = wall_clock64();
+        if (!known) {
+          L.seen_base = g;
+          L.seen = found;
+        }
+        L.ptr = c.rings + (uint64_t)pe_index() * c.ring_stride +
+                (pos & (c.ring_bytes - 1));
+      }
       return CMD_INBOX;
     }
-    if (ps->n_waits > 0) {
-      for (int i = 0; i < ASYNC_WAIT_MAX; i++) {
-        AsyncWait& w = ps->waits[i];
-        if (!w.valid || !wait_satisfied(w)) continue;
-        L.t_found = wall_clock64();
-        fence_acquire();
-        w.valid = 0;
-        ps->n_waits--;
-        L.arg = w.proxy;
-        L.n = w.idx;
-        L.pos = (uint64_t)w.ep;
-        return CMD_ASYNC;
-      }
-    }
-    if (ld_relaxed(&c.ctl[CTL_TERM]) != 0) return CMD_EXIT;
-    if ((spins & 255) == 255) {
-      if (*c.host_abort) {
-        raise_error(ERR_HOST_ABORT, 0);
-        return CMD_EXIT;
-      }
-      ps->stats.idle_polls++;
-    }
+    if (l == 0) cmd = poll_rest(spins);
+    cmd = __builtin_amdgcn_readfirstlane(cmd);
+    if (cmd >= 0) return cmd;
     __builtin_amdgcn_s_sleep(1);
   }
 }
@@ -550,10 +721,10 @@ __device__ __noinline__ void process_inbox() {
   if (threadIdx.x == 0) {
     flush_publish();
     wave_drain();
-    ps->read_pos += slot;
-    st_relaxed(&c.heads[(uint64_t)pe_index() * 16], ps->read_pos);
-    if (ok) ps->stats.delivered++;
-    ps->stats.overhead_ticks += wall_clock64() - lds().t_found;
+    lds().read_pos += slot;
+    st_relaxed(&c.heads[(uint64_t)pe_index() * 16], lds().read_pos);
+    if (ok) lds().stats.delivered++;
+    lds().stats.overhead_ticks += wall_clock64() - lds().t_found;
   }
 }
 
@@ -569,8 +740,8 @@ __device__ __noinline__ void process_revived() {
     if (ok) {
       d.state = 0;
       ps->n_deferred--;
-      ps->stats.delivered++;
-      ps->stats.revived++;
+      lds().stats.delivered++;
+      lds().stats.revived++;
       if (ps->n_deferred == 0) {
         ps->arena_used = 0;
         ps->hw = 0;
@@ -595,8 +766,8 @@ __device__ __noinline__ void process_async() {
   __syncthreads();
   if (threadIdx.x == 0) {
     flush_publish();
-    ps->stats.delivered++;
-    ps->stats.overhead_ticks += wall_clock64() - L.t_found;
+    lds().stats.delivered++;
+    lds().stats.overhead_ticks += wall_clock64() - L.t_found;
   }
 }
 
@@ -631,7 +802,10 @@ __device__ __noinline__ void run_work() {
 // is told to stop.
 __device__ __noinline__ bool pe_step() {
   Lds& L = lds();
-  if (threadIdx.x == 0) L.cmd = poll_next();
+  if (threadIdx.x < kAhead) {
+    const int found = poll_next();
+    if (threadIdx.x == 0) L.cmd = found;
+  }
   __syncthreads();
   const int cmd = L.cmd;
   if (cmd == CMD_EXIT) return false;
@@ -651,7 +825,10 @@ __device__ __noinline__ bool pe_step() {
 // the kernel's register total on top of the hook's.
 __device__ __noinline__ void pe_loop() {
   while (pe_step()) {
-    run_work();
+    // (a request is made before the turn's last barrier.  Tested here, not in
+    // run_work, whose entry parks some 190 registers of every lane: called
+    // after each message, it made that 10 us of the 12 that a message took.)
+    if (lds().has_work) run_work();
     __syncthreads();
   }
 }
@@ -704,7 +881,9 @@ __device__ void pe_begin() {
 #endif
     PeState* ps = pe_state();
     const uint64_t t = ld_relaxed(&g_ctx.tails[(uint64_t)pe_index() * 16]);
-    ps->read_pos = t;
+    lds().read_pos = t;
+    lds().seen_base = 0;
+    lds().seen = 0;
     st_relaxed(&g_ctx.heads[(uint64_t)pe_index() * 16], t);
     ps->table.count = 0;
     ps->heap_used = 0;
@@ -718,12 +897,16 @@ __device__ void pe_begin() {
     for (int i = 0; i < ASYNC_WAIT_MAX; i++) ps->waits[i].valid = 0;
     lds().n_pend = 0;
     lds().has_work = 0;
-    for (int i = 0; i < CHARMING_DEFERRED_MAX; i++) ps->deferred[i].state = 0;
-    ps->stats = Stats{};
+    lds().stats = Stats{};
     ps->n_user_free = g_ctx.user_bytes ? 1 : 0;
     ps->user_free[0].offset = 0;
     ps->user_free[0].size = g_ctx.user_bytes;
   }
+#ifdef CHARMING_GPU_LEVEL
+  if (blockIdx.x == 0)
+#endif
+    for (int i = threadIdx.x; i < CHARMING_DEFERRED_MAX; i += blockDim.x)
+      pe_state()->deferred[i].state = 0;
   __syncthreads();
 }
 
@@ -875,14 +1058,14 @@ __device__ void gpu_finish() {
   flush_publish();
   if (L.g_kind == CMD_INBOX) {
     wave_drain();
-    ps->read_pos += L.g_slot;
-    st_relaxed(&g_ctx.heads[(uint64_t)pe_index() * 16], ps->read_pos);
+    L.read_pos += L.g_slot;
+    st_relaxed(&g_ctx.heads[(uint64_t)pe_index() * 16], L.read_pos);
   } else if (L.g_kind == CMD_REVIVED) {
     DeferredEntry& d = ps->deferred[L.arg];
     if (L.g_run) {
       d.state = 0;
       ps->n_deferred--;
-      ps->stats.revived++;
+      lds().stats.revived++;
       if (ps->n_deferred == 0) {
         ps->arena_used = 0;
         ps->hw = 0;
@@ -891,7 +1074,7 @@ __device__ void gpu_finish() {
       d.state = 1;  // refnum moved on again: stay deferred
     }
   }
-  if (L.g_run) ps->stats.delivered++;
+  if (L.g_run) lds().stats.delivered++;
 }
 
 __device__ __noinline__ void gpu_pe_loop() {
@@ -1150,6 +1333,10 @@ __device__ __noinline__ void pe_run() {
 #else
   pe_loop();
 #endif
+#ifdef CHARMING_GPU_LEVEL
+  if (blockIdx.x == 0)
+#endif
+    if (threadIdx.x == 0) pe_state()->stats = lds().stats;
   grid_barrier();
 }
 
