@@ -27,6 +27,17 @@ __host__ __device__ inline void split_extent(int len, int n, int r, int* start,
   *size = (r == n - 1) ? len - b * (n - 1) : b;
 }
 
+// Workgroup-collective: the sum of every thread's v, in thread 0.
+__device__ inline uint64_t block_sum(uint64_t v) {
+  __shared__ uint64_t part[16];
+  for (int off = 32; off >= 1; off >>= 1) v += __shfl_down(v, off, 64);
+  if (__lane_id() == 0) part[threadIdx.x / 64] = v;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int w = 1; w < (int)(blockDim.x / 64); w++) v += part[w];
+  return v;
+}
+
 struct PersistentState;  // defined by the message-driven form
 
 // Two pinned buffers through which a grid goes to the host, made at the first

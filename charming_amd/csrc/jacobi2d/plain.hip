@@ -68,17 +68,6 @@ __device__ inline int xcd_logical_block(int n) {
   return (i % 8) * per + i / 8;
 }
 
-// Workgroup-collective: the sum of every thread's v, in thread 0.
-__device__ inline uint64_t block_sum(uint64_t v) {
-  __shared__ uint64_t part[16];
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_down(v, off, 64);
-  if (__lane_id() == 0) part[threadIdx.x / 64] = v;
-  __syncthreads();
-  if (threadIdx.x == 0)
-    for (int w = 1; w < (int)(blockDim.x / 64); w++) v += part[w];
-  return v;
-}
-
 // Workgroup-collective: the exact sum of every thread's acc is added to out.
 __device__ inline void block_add_u128(uint64_t* out, u128acc acc) {
   __shared__ u128acc part[16];
