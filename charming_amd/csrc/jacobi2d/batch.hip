@@ -646,7 +646,7 @@ __device__ void admit(const EngineDesc& E, uint64_t idx, Request* s_req) {
     ast(&p.fix_sweeps, 0u);
     for (int i = 0; i < 2; i++) {
       ast(&p.round_tiles[i], 0u);
-      for (int j = 0; j < 8; j++) {
+      for (int j = 0; j < 16; j++) {
         ast(&p.res[i][j][0], 0ull);
         ast(&p.res[i][j][1], 0ull);
         ast((uint64_t*)&p.resd[i][j], 0ull);
