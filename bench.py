@@ -17,9 +17,10 @@ per cell-update (read u_k once, write u_{k+D} once per D updates).
 `roofline.achieved` is that figure times the launch's cell-updates over its
 HIP-event duration; `roofline.traffic` is the bytes the memory system really
 moved (rocprof FETCH_SIZE + WRITE_SIZE, calibrated), beside its ratio to the
-minimum.  At sixteen fused sweeps the launch is bound by vector-ALU issue
-rather than by HBM (profiles/sq_valu_jacobi2d_16384_persistent.md), so the
-HBM fraction is not the binding one.  The 16 B-per-update rate of the
+minimum.  At sixteen fused sweeps the launch keeps the vector ALU busy 69 %
+of its issue slots and the memory system at four fifths of the copy rate
+(profiles/sq_valu_jacobi2d_16384_persistent.md), so the HBM fraction alone
+is not the binding one.  The 16 B-per-update rate of the
 unfused sweep is reported separately (`gbs_at_16B_per_update`), and the
 one-sweep-per-exchange persistent form, which moves 16 B per update, is
 measured beside the plain forms.

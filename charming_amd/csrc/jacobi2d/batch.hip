@@ -1469,9 +1469,9 @@ static int batch_once(const chm_batch_problem* probs, int n,
                       const int* blocks, BatchOut out) {
   if (n < 1 || n > (int)kMaxSlots)
     return fail(CHM_E_INVALID, "%d problems (1..%u)", n, kMaxSlots);
-  // (default 512 threads: sixteen sweeps per round, 105-108 ms for the
-  // 512-problem batch at the size rule's tiles, against 123-124 ms at 1024
-  // threads and eight sweeps per round, and 136 ms at 256 threads)
+  // (default 512 threads: sixteen sweeps per round by groups of waves, 68-71
+  // ms for the 512-problem batch at pick_blocks' tiles, against 123-124 ms at
+  // 1024 threads and eight sweeps per round, and 136 ms at 256 threads)
   const int threads = cfg && cfg->wg_threads ? cfg->wg_threads : 512;
   const int block = cfg ? cfg->block : 0;
   const int nc = cfg && cfg->panel_chunks ? cfg->panel_chunks : 1;

@@ -465,8 +465,8 @@ __device__ void sweepD_dispatch(int steps, const double* in, double* out,
 // Sixteen fused sweeps of the whole block (halos sixteen deep) by groups of
 // four waves (pipeline.h): every full round but the last of a solve, unless
 // the caller asked for bands of the window pass.  16384^2 x 1000, 16 x 16
-// chares: 118-119 -> 90-91 ms per solve; 4096^2 x 200, 8 x 8 chares:
-// 10.9 -> 6.4 ms.  Other depths and the last round (its residual) run the
+// chares: 118-119 -> 90-91 ms per solve (80-82 with the scheduler's messages
+// at 2 us each); 4096^2 x 200, 8 x 8 chares: 10.9 -> 6.4 ms (5.1).  Other depths and the last round (its residual) run the
 // window pass.
 __device__ __noinline__ void chare_pipe(const double* in, double* out,
                                         int64_t P, int bw, int bh,
@@ -1105,7 +1105,7 @@ int persistent_create(Handle* h) {
     chm_config cfg;
     memset(&cfg, 0, sizeof(cfg));
     // watchdog: generous for the largest grids this form is used on
-    // (16384^2 x 1000 sweeps takes about a second)
+    // (16384^2 x 1000 sweeps takes 0.08 seconds)
     cfg.timeout_s = 120.0;
     int rc = chm_init(0, nullptr, &cfg);
     if (rc == CHM_E_NOMEM && DevCache::get().release())
