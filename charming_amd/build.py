@@ -41,6 +41,7 @@ LIBS = [
     ("libchm_pingpong.so", ["examples/pingpong.hip"], ["charming_amd"]),
     ("libchm_async_wait.so", ["examples/async_wait.hip"], ["charming_amd"]),
     ("libchm_failure.so", ["examples/failure.hip"], ["charming_amd"]),
+    ("libchm_broadcast.so", ["examples/broadcast.hip"], ["charming_amd"]),
     # GPU-level builds (one PE spanning every workgroup): SRC@gpu is SRC
     # compiled with CHARMING_GPU_LEVEL
     ("libchm_hello_gpu.so", ["examples/hello.hip@gpu"], ["charming_amd"]),
@@ -138,6 +139,7 @@ STACK_BYTES = 4096
 CHARE_PROGRAMS = ["jacobi2d/persistent.hip", "examples/hello.hip",
                   "examples/refnum.hip", "examples/pingpong.hip",
                   "examples/async_wait.hip", "examples/failure.hip",
+                  "examples/broadcast.hip",
                   "examples/hello.hip@gpu", "examples/pingpong.hip@gpu"]
 
 

@@ -50,7 +50,7 @@ constexpr int kMaxPending = 16;
 // published together share one acquire and the lines it brings back.  16
 // words are one or two cache lines.
 constexpr int kAhead = 16;
-constexpr uint64_t kSmallPayload = 64;  // a lane's own copy, see send_all
+constexpr uint64_t kSmallPayload = 64;  // copied by single lanes, see send_all
 enum : int { CMD_EXIT = 0, CMD_INBOX = 1, CMD_REVIVED = 2, CMD_ASYNC = 3 };
 
 // Workgroup-shared scratch used to broadcast thread 0's decisions.  The
@@ -88,6 +88,7 @@ struct Lds {
   uint64_t* pend_addr[kMaxPending];
   uint64_t pend_tag[kMaxPending];
   uint32_t order[CHARMING_DEFERRED_MAX];
+  char small[kSmallPayload];  // thread 0's payload of a broadcast (send_all)
 };
 static __shared__ Lds s_lds;
 
@@ -414,8 +415,10 @@ __device__ void send_lanes(bool mine, int dst, int idx, const char* from,
 #endif
 
 // Workgroup-collective: one message with thread 0's payload for entry method
-// ep of each of the n chares, chare i on PE i (n <= n_pes).  False, with
-// nothing sent, where the payload is more than a lane should copy.
+// ep of each of the n chares, chare i on PE i (n <= n_pes).  Thread 0 alone
+// reads the payload: it may lie in that thread's own memory, where the same
+// address means another place to every other lane.  False, with nothing sent,
+// where the payload is more than a lane should copy.
 __device__ __noinline__ bool send_all(int chare_id, int ep, const void* buf,
                                       uint64_t payload, int n) {
 #ifdef CHARMING_GPU_LEVEL
@@ -429,6 +432,8 @@ __device__ __noinline__ bool send_all(int chare_id, int ep, const void* buf,
     L.snd.chare_id = chare_id;
     L.snd.ep = ep;
     L.snd.refnum = -1;
+    if (payload <= kSmallPayload)
+      for (uint64_t k = 0; k < payload; k++) L.small[k] = ((const char*)buf)[k];
   }
   __syncthreads();
   const uint64_t bytes = L.snd.payload;
@@ -438,7 +443,7 @@ __device__ __noinline__ bool send_all(int chare_id, int ep, const void* buf,
     return false;
   for (int base = 0; base < n; base += blockDim.x) {
     const int i = base + (int)threadIdx.x;
-    send_lanes(i < n, i, i, (const char*)L.snd.buf, bytes);
+    send_lanes(i < n, i, i, L.small, bytes);
   }
   __syncthreads();
   return true;
