@@ -52,3 +52,37 @@ def test_thread_zeros_payload_counts(capfd, pes, count, nbytes):
     assert (f"{count} payloads of {nbytes} bytes to {pes} chares, 0 wrong"
             in out), out[-2000:]
     assert int(st["delivered"]) == 1 + pes * count + pes
+
+
+RING = dict(CHM_RING_BYTES=65536, CHM_MAX_MSG_BYTES=32768)
+
+
+def _still_works(capfd):
+    rc, out, err, st = _run(capfd, ["word", 2, 12], CHM_N_PES=9)
+    assert rc == 0 and "12 bytes to 9 chares, 0 wrong" in out, err[-2000:]
+
+
+@pytest.mark.parametrize("pes,nbytes", [(3, 8), (70, 24)])
+def test_lanes_wait_for_room(capfd, pes, nbytes):
+    # chare 1's PE is busy and three quarters of its inbox taken: about 270 of
+    # the 400 broadcasts fit, each later one waits for its one late lane
+    rc, out, err, st = _run(capfd, ["full", 400, nbytes], CHM_N_PES=pes, **RING)
+    assert rc == 0, err[-2000:]
+    assert f"400 payloads of {nbytes} bytes to {pes} chares, 0 wrong" in out
+    assert int(st["send_spins"]) > 0
+
+
+def test_waiting_lane_gives_up_at_the_spin_limit(capfd):
+    rc, out, err, st = _run(capfd, ["full", 400, 8], CHM_N_PES=70,
+                            CHM_SPIN_LIMIT=2000, **RING)
+    assert rc == 1
+    assert "device error 8 (send spin limit reached" in err, err[-2000:]
+    assert int(st["send_spins"]) >= 2000
+    _still_works(capfd)
+
+
+def test_own_inbox_full_fails_at_once(capfd):
+    # 1024 messages of 64 bytes fill the sender's own ring
+    rc, out, err, st = _run(capfd, ["self", 1100, 8], CHM_N_PES=3, **RING)
+    assert rc == 1 and st["error"] == "2", err[-2000:]
+    _still_works(capfd)
