@@ -26,6 +26,7 @@
 #include <thread>
 #include <vector>
 
+#include "cell_share.h"
 #include "dev_cache.h"
 #include "engine_dev.h"
 #include "jacobi2d_internal.h"
@@ -984,13 +985,15 @@ __global__ void init_queues(uint64_t* cells, uint64_t n_cells, uint32_t qcap) {
 }
 
 // Host-launched seeding of whole problems: u_0 in every array (rows 1-depth ..
-// H+depth), padding 0.  A wave takes a row at a time (no division per cell).
+// H+depth), padding 0.  A wave takes a row, or part of one, at a time.
 __device__ inline void init_rows(const Request& r) {
   const int d = r.depth, waves = blockDim.x / 64;
-  for (int i = 1 - d + (int)(blockIdx.x * waves + threadIdx.x / 64);
-       i <= r.H + d; i += gridDim.x * waves) {
+  const jac::CellShare s = jac::cell_share(
+      r.H + 2 * d, (int)r.pitch, blockIdx.x * waves + threadIdx.x / 64,
+      gridDim.x * waves, 64, threadIdx.x & 63);
+  for (int i = 1 - d + s.row; i <= r.H + d; i += s.row_step) {
     const int64_t o = (int64_t)i * r.pitch;
-    for (int64_t e = threadIdx.x & 63; e < r.pitch; e += 64) {
+    for (int e = s.col; e < r.pitch; e += s.col_step) {
       const int64_t j = e - kColOff;
       const double v = (j >= 1 - d && j <= r.W + d) ? u0_cell(r, i, j) : 0.0;
       r.a[o + e] = v;

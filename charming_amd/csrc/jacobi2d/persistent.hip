@@ -42,6 +42,7 @@ __device__ void jacobi_work(void* token);
 #include <algorithm>
 #include <vector>
 
+#include "cell_share.h"
 #include "dev_cache.h"
 #include "jacobi2d_internal.h"
 #include "pipeline.h"
@@ -1001,10 +1002,11 @@ __global__ void init_chares_kernel(JacobiDesc d, uint64_t seed, int mode,
   double* a = d.arena + (int64_t)(2 * c) * d.chare_elems;
   double* b = a + d.chare_elems;
   const double ring = (mode == CHM_INIT_REFERENCE) ? 10.0 : boundary;
-  // (a row per workgroup at a time: no 64-bit division per cell)
-  for (int row = blockIdx.x; row < g.bh + 2 * kHaloRows; row += gridDim.x) {
+  const CellShare s = cell_share(g.bh + 2 * kHaloRows, (int)P, blockIdx.x,
+                                 gridDim.x, blockDim.x, threadIdx.x);
+  for (int row = s.row; row < g.bh + 2 * kHaloRows; row += s.row_step) {
     const int64_t i = row - (kHaloRows - 1), gi = g.row0 + i;
-    for (int64_t e = threadIdx.x; e < P; e += blockDim.x) {
+    for (int e = s.col; e < P; e += s.col_step) {
       const int64_t j = e - kColOff, gj = g.col0 + j;
       double v = 0.0;
       if (j >= 1 - kHaloRows && j <= g.bw + kHaloRows && gi >= 0 &&
@@ -1031,9 +1033,11 @@ __global__ void hash_chares_kernel(JacobiDesc d, int parity, int r0, int r1,
       d.arena + (int64_t)(2 * c + parity) * d.chare_elems + (kHaloRows - 1) * P;
   const int lr0 = max(r0, g.row0 + 1), lr1 = min(r1, g.row0 + 1 + g.bh);
   const int lc0 = max(c0, g.col0 + 1), lc1 = min(c1, g.col0 + 1 + g.bw);
+  const CellShare s = cell_share(lr1 - lr0, lc1 - lc0, blockIdx.x, gridDim.x,
+                                 blockDim.x, threadIdx.x);
   uint64_t h = 0;
-  for (int gi = lr0 + blockIdx.x; gi < lr1; gi += gridDim.x)
-    for (int gj = lc0 + threadIdx.x; gj < lc1; gj += blockDim.x)
+  for (int gi = lr0 + s.row; gi < lr1; gi += s.row_step)
+    for (int gj = lc0 + s.col; gj < lc1; gj += s.col_step)
       h += hash_cell(gi, gj, a[(gi - g.row0) * P + kColOff + gj - g.col0]);
   h = block_sum(h);
   if (threadIdx.x == 0 && h)

@@ -14,6 +14,7 @@
 #include <new>
 #include <vector>
 
+#include "cell_share.h"
 #include "dev_cache.h"
 #include "jacobi2d_internal.h"
 #include "pipeline.h"
@@ -40,10 +41,12 @@ __global__ void init_global_kernel(double* a, double* b, int W, int H,
                                    int64_t P, uint64_t seed, int mode,
                                    double boundary) {
   const double ring = (mode == CHM_INIT_REFERENCE) ? 10.0 : boundary;
-  // (a row per workgroup at a time: an index per cell costs two 64-bit
-  // divisions, which took longer than the stores)
-  for (int i = blockIdx.x; i < H + 2; i += gridDim.x)
-    for (int64_t e = threadIdx.x; e < P; e += blockDim.x) {
+  // (an index per cell would cost two 64-bit divisions, which took longer than
+  // the stores)
+  const CellShare s = cell_share(H + 2, (int)P, blockIdx.x, gridDim.x,
+                                 blockDim.x, threadIdx.x);
+  for (int i = s.row; i < H + 2; i += s.row_step)
+    for (int e = s.col; e < P; e += s.col_step) {
       const int64_t j = e - kColOff;
       double v = 0.0;
       if (j >= 0 && j <= W + 1) {
@@ -123,9 +126,11 @@ __global__ void __launch_bounds__(512)
 // Order-independent hash over interior rows [r0,r1) x cols [c0,c1).
 __global__ void hash_global_kernel(const double* g, int64_t P, int r0, int r1,
                                    int c0, int c1, uint64_t* out) {
+  const CellShare s = cell_share(r1 - r0, c1 - c0, blockIdx.x, gridDim.x,
+                                 blockDim.x, threadIdx.x);
   uint64_t h = 0;
-  for (int i = r0 + blockIdx.x; i < r1; i += gridDim.x)
-    for (int j = c0 + threadIdx.x; j < c1; j += blockDim.x)
+  for (int i = r0 + s.row; i < r1; i += s.row_step)
+    for (int j = c0 + s.col; j < c1; j += s.col_step)
       h += hash_cell(i, j, g[i * P + kColOff + j]);
   h = block_sum(h);
   if (threadIdx.x == 0 && h)
@@ -136,9 +141,11 @@ __global__ void hash_global_kernel(const double* g, int64_t P, int r0, int r1,
 __global__ void residual_global_kernel(const double* a, const double* b,
                                        int W, int H, int64_t P,
                                        uint64_t* out) {
+  const CellShare s =
+      cell_share(H, W, blockIdx.x, gridDim.x, blockDim.x, threadIdx.x);
   u128acc acc = {0, 0};
-  for (int i = 1 + blockIdx.x; i <= H; i += gridDim.x)
-    for (int j = 1 + threadIdx.x; j <= W; j += blockDim.x) {
+  for (int i = 1 + s.row; i <= H; i += s.row_step)
+    for (int j = 1 + s.col; j <= W; j += s.col_step) {
       const int64_t o = i * P + kColOff + j;
       acc_add(acc, res_term(a[o], b[o]));
     }
@@ -401,9 +408,11 @@ __global__ void begin_noalloc_kernel(const double* src, double* dst, int W,
 // acc[3] counts workgroups.
 __global__ void end_noalloc_kernel(const double* g, double* copy, int W, int H,
                                    int64_t P, uint64_t* acc, uint64_t* out) {
+  const CellShare s =
+      cell_share(H, W, blockIdx.x, gridDim.x, blockDim.x, threadIdx.x);
   uint64_t h = 0;
-  for (int i = 1 + blockIdx.x; i <= H; i += gridDim.x)
-    for (int j = 1 + threadIdx.x; j <= W; j += blockDim.x) {
+  for (int i = 1 + s.row; i <= H; i += s.row_step)
+    for (int j = 1 + s.col; j <= W; j += s.col_step) {
       const int64_t o = i * P + kColOff + j;
       const double v = g[o];
       h += hash_cell(i, j, v);
@@ -578,7 +587,7 @@ static int solve_noalloc(double* grid, int W, int H, int iters,
                            L.n_tiles, L.n_blocks);
     }
   }
-  end_noalloc_kernel<<<std::min(1024, H), 256, 0, stream>>>(
+  end_noalloc_kernel<<<cell_wgs(H, W, 256, 1024), 256, 0, stream>>>(
       g[cur], cur ? grid : nullptr, W, H, P, acc, out3);
   CHM_TRY_HIP(hipGetLastError());
   return CHM_OK;
