@@ -12,11 +12,11 @@
 #include <algorithm>
 #include <mutex>
 #include <new>
-#include <vector>
 
 #include "cell_share.h"
 #include "dev_cache.h"
 #include "jacobi2d_internal.h"
+#include "noalloc_plan.h"
 #include "pipeline.h"
 
 namespace chm {
@@ -509,32 +509,6 @@ static void launch_pass(int depth, const double* in, double* out, int W, int H,
 #undef CHM_PASS
 }
 
-// Sweeps per launch of `iters` sweeps whose last one is a launch of its own
-// (it leaves u_{iters-1} for the residual): sixteen, then what is left in
-// fours, then single sweeps.  An even number of launches ends in the array
-// it began in, so of an odd one a pass is split, which costs less than the
-// copy back.  Grids lower than sixteen rows are swept one at a time (a pass
-// needs the ring's rows that far apart).
-static std::vector<int> noalloc_launches(int H, int iters) {
-  std::vector<int> l;
-  int left = iters - 1;
-  while (H >= 16 && left >= 4) {
-    l.push_back(std::min(16, left / 4 * 4));
-    left -= l.back();
-  }
-  const size_t passes = l.size();
-  for (; left > 0; left--) l.push_back(1);
-  l.push_back(1);
-  if (l.size() % 2 && passes > 0 && l[passes - 1] > 4) {
-    l[passes - 1] -= 4;
-    l.insert(l.begin() + passes, 4);
-  } else if (l.size() % 2 && passes > 0 && l[0] > 4) {
-    l[0] -= 4;
-    l.insert(l.begin() + 1, 4);
-  }
-  return l;
-}
-
 static int solve_noalloc(double* grid, int W, int H, int iters,
                          hipStream_t stream, uint64_t* out3) {
   if (!grid || !out3) return fail(CHM_E_INVALID, "null grid or output");
@@ -573,9 +547,9 @@ static int solve_noalloc(double* grid, int W, int H, int iters,
   double* g[2] = {grid, other};
   int cur = 0;
   if (iters > 0) {
-    const std::vector<int> launches = noalloc_launches(H, iters);
-    for (size_t i = 0; i < launches.size(); i++, cur ^= 1) {
-      if (i + 1 == launches.size())
+    const NoallocPlan launches = noalloc_plan(H, iters);
+    for (int i = 0; i < launches.n; i++, cur ^= 1) {
+      if (i + 1 == launches.n)
         plain_step_residual_kernel<<<R.grid, R.block, 0, stream>>>(
             g[cur], g[cur ^ 1], W, H, P, R.band_rows, R.n_panels, R.n_tiles,
             R.n_blocks, acc + 1);
