@@ -67,9 +67,11 @@ struct Handle {
   GridReader* reader;
 };
 
-// Launches, on the problem's stream, what writes rows [row, row + rows) of
-// the grid, ring included, to `dst` (W + 2 cells a row).
-void persistent_gather(Handle* h, double* dst, int row, int rows);
+// Launches, on the problem's stream, what writes rows [row, row + rows) x
+// columns [col, col + cols) of the grid, ring included, to `dst` (cols cells
+// a row).
+void persistent_gather(Handle* h, double* dst, int row, int rows, int col,
+                       int cols);
 
 // Forms implemented in other translation units.
 int persistent_create(Handle* h);

@@ -1,5 +1,5 @@
 // The launches of a no-alloc solve, as counts: a list of them would grow with
-// the sweeps (16 GB for 2^31 single sweeps of a low grid) and could throw
+// the sweeps (8 GB for 2^31 single sweeps of a low grid) and could throw
 // across the C entry.
 #pragma once
 

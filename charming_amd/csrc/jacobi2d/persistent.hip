@@ -1044,13 +1044,14 @@ __global__ void hash_chares_kernel(JacobiDesc d, int parity, int r0, int r1,
     __hip_atomic_fetch_add(out, h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Rows [row, row + rows) of the grid, ring included, from the chares' blocks
-// to `out` (pinned host memory: bound by the link, 256 cells of a row to a
-// workgroup are whole lines but for their ends).
+// Rows [row, row + rows) x columns [col, col + cols) of the grid, ring
+// included, from the chares' blocks to `out` (pinned host memory: bound by the
+// link, 256 cells of a row to a workgroup are whole lines but for their ends).
 __global__ void gather_chares_kernel(JacobiDesc d, int parity, double ring,
-                                     int row, int rows, double* out) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= d.W + 2) return;
+                                     int row, int rows, int col, int cols,
+                                     double* out) {
+  const int jo = blockIdx.x * blockDim.x + threadIdx.x, j = col + jo;
+  if (jo >= cols) return;
   const int cx = max(0, min((j - 1) / (d.W / d.cc), d.cc - 1));
   for (int k = blockIdx.y; k < rows; k += gridDim.y) {
     const int i = row + k;
@@ -1062,7 +1063,7 @@ __global__ void gather_chares_kernel(JacobiDesc d, int parity, double ring,
                   (kHaloRows - 1 + i - g.row0) * chare_pitch(g.bw) + kColOff +
                   j - g.col0];
     }
-    out[(int64_t)k * (d.W + 2) + j] = v;
+    out[(int64_t)k * cols + jo] = v;
   }
 }
 
@@ -1270,12 +1271,13 @@ int persistent_hash_region(Handle* h, int r0, int r1, int c0, int c1,
   return CHM_OK;
 }
 
-void persistent_gather(Handle* h, double* dst, int row, int rows) {
+void persistent_gather(Handle* h, double* dst, int row, int rows, int col,
+                       int cols) {
   const double ring =
       (h->prob.init_mode == CHM_INIT_REFERENCE) ? 10.0 : h->prob.boundary;
-  gather_chares_kernel<<<dim3((h->W + 2 + 255) / 256, std::min(rows, 4096)),
-                         256, 0, h->stream>>>(h->ps->desc, h->cur, ring, row,
-                                              rows, dst);
+  gather_chares_kernel<<<dim3((cols + 255) / 256, std::min(rows, 4096)), 256,
+                         0, h->stream>>>(h->ps->desc, h->cur, ring, row, rows,
+                                         col, cols, dst);
 }
 
 int persistent_chare_count(Handle* h, int* n) {

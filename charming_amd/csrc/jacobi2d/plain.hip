@@ -18,6 +18,7 @@
 #include "jacobi2d_internal.h"
 #include "noalloc_plan.h"
 #include "pipeline.h"
+#include "read_plan.h"
 
 namespace chm {
 namespace jac {
@@ -26,13 +27,14 @@ namespace jac {
 // kernels over one (H+2) x P array
 // ----------------------------------------------------------------------------
 
-// Rows [row, row + rows) of a grid to `out` (pinned host memory).
-__global__ void gather_rows_kernel(const double* a, int64_t P, int W, int row,
-                                   int rows, double* out) {
+// Rows [row, row + rows) x columns [col, col + cols) of a grid to `out` (pinned
+// host memory).
+__global__ void gather_rows_kernel(const double* a, int64_t P, int row,
+                                   int rows, int col, int cols, double* out) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= W + 2) return;
+  if (j >= cols) return;
   for (int k = blockIdx.y; k < rows; k += gridDim.y)
-    out[(int64_t)k * (W + 2) + j] = a[(row + k) * P + kColOff + j];
+    out[(int64_t)k * cols + j] = a[(row + k) * P + kColOff + col + j];
 }
 
 // u_0: seeded interior (or 0 in the reference init), ring = boundary (or 10),
@@ -568,46 +570,41 @@ static int solve_noalloc(double* grid, int W, int H, int iters,
 }
 
 // The grid to the caller's memory, through two pinned buffers: a kernel packs
-// a piece of about kReadBytes over the link while the host copies the one
-// before out.  A copy command straight to pageable memory pins and unpins it
-// first, once for every row block of a strided one: 3001 x 1777 in 256 chares
-// took 190 ms and takes 2.7; 1500 x 1100 took 7.8 ms, now 0.5.  The host's
-// copy, with its page faults, is what is left (14 GB/s into huge pages).
-constexpr size_t kReadBytes = 1 << 20;
-
+// a piece over the link while the host copies the one before out.  A copy
+// command straight to pageable memory pins and unpins it first, once for every
+// row block of a strided one: 3001 x 1777 in 256 chares took 190 ms and takes
+// 2.7; 1500 x 1100 took 7.8 ms, now 0.5.  The host's copy, with its page
+// faults, is what is left (14 GB/s into huge pages).
 static int read_rows(Handle* h, double* out) {
-  const size_t row_bytes = (size_t)(h->W + 2) * sizeof(double);
-  const int n_rows = h->H + 2;
-  const int step = (int)std::min<size_t>(
-      n_rows, std::max<size_t>(1, kReadBytes / row_bytes));
-  const int n = (n_rows + step - 1) / step;
+  const ReadPlan p = read_plan(h->H + 2, h->W + 2);
   GridReader* r = h->reader;
   std::lock_guard<std::mutex> lock(r->mu);
-  for (int i = 0; i < std::min(n, 2); i++) {
+  for (int i = 0; i < std::min(p.n, 2); i++) {
     if (!r->done[i])
       CHM_TRY_HIP(hipEventCreateWithFlags(&r->done[i],
                                           hipEventDisableTiming));
     if (!r->buf[i])
-      CHM_TRY_HIP(hipHostMalloc(&r->buf[i], step * row_bytes, 0));
+      CHM_TRY_HIP(hipHostMalloc(
+          &r->buf[i], (size_t)p.rows * p.cols * sizeof(double), 0));
   }
   auto pack = [&](int k) {
-    const int row = k * step, rows = std::min(step, n_rows - row);
+    const int rows = p.rows_of(k), cols = p.cols_of(k);
     if (h->form == CHM_FORM_PERSISTENT)
-      persistent_gather(h, r->buf[k & 1], row, rows);
+      persistent_gather(h, r->buf[k & 1], p.row(k), rows, p.col(k), cols);
     else
-      gather_rows_kernel<<<dim3((h->W + 2 + 255) / 256, std::min(rows, 4096)),
-                           256, 0, h->stream>>>(h->grid[h->cur], h->P, h->W,
-                                                row, rows, r->buf[k & 1]);
+      gather_rows_kernel<<<dim3((cols + 255) / 256, std::min(rows, 4096)), 256,
+                           0, h->stream>>>(h->grid[h->cur], h->P, p.row(k),
+                                           rows, p.col(k), cols, r->buf[k & 1]);
     CHM_TRY_HIP(hipGetLastError());
     CHM_TRY_HIP(hipEventRecord(r->done[k & 1], h->stream));
     return CHM_OK;
   };
   CHM_TRY(pack(0));
-  for (int k = 0; k < n; k++) {
-    if (k + 1 < n) CHM_TRY(pack(k + 1));
+  for (int k = 0; k < p.n; k++) {
+    if (k + 1 < p.n) CHM_TRY(pack(k + 1));
     CHM_TRY_HIP(hipEventSynchronize(r->done[k & 1]));
-    const int row = k * step, rows = std::min(step, n_rows - row);
-    memcpy((char*)out + row * row_bytes, r->buf[k & 1], rows * row_bytes);
+    memcpy(out + p.first(k), r->buf[k & 1],
+           (size_t)p.rows_of(k) * p.cols_of(k) * sizeof(double));
   }
   return CHM_OK;
 }
