@@ -1853,7 +1853,7 @@ using namespace chm::eng;
 extern "C" {
 
 int chm_jacobi2d_release_memory(void) {
-  (void)jac::DevCache::get().release();
+  (void)jac::DevCache::get().release(jac::DevCache::kAllDevices);
   return CHM_OK;
 }
 

@@ -29,6 +29,8 @@ struct DevBlock {
 
 class DevCache {
  public:
+  static constexpr int kAllDevices = -1;
+
   // (never destroyed: its blocks go with the process)
   static DevCache& get() {
     static DevCache* c = new DevCache;
@@ -58,11 +60,11 @@ class DevCache {
     return alloc(&b->p, bytes);
   }
 
-  // hipMalloc, with what is kept given back if it fails.
+  // hipMalloc, with what is kept on the current device given back if it fails.
   template <class T>
   hipError_t alloc(T** p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
-    if (e == hipSuccess || !release()) return e;
+    if (e == hipSuccess || !release_current()) return e;
     (void)hipGetLastError();
     return hipMalloc(p, bytes);
   }
@@ -104,16 +106,25 @@ class DevCache {
     for (int i = 0; i < n_out; i++) (void)hipFree(out[i]);
   }
 
-  // Gives everything back; false if nothing was kept.
-  bool release() {
+  // Gives back what is kept on `dev` (kAllDevices: on any); false if nothing
+  // was.
+  bool release(int dev) {
     void* out[kBlocks];
     int n_out = 0;
     {
       std::lock_guard<std::mutex> lk(mu_);
-      while (n_ > 0) out[n_out++] = kept_[--n_].b.p;
+      for (int i = n_ - 1; i >= 0; i--) {
+        if (dev != kAllDevices && kept_[i].b.dev != dev) continue;
+        out[n_out++] = kept_[i].b.p;
+        kept_[i] = kept_[--n_];
+      }
     }
     for (int i = 0; i < n_out; i++) (void)hipFree(out[i]);
     return n_out > 0;
+  }
+  bool release_current() {
+    int dev = 0;
+    return hipGetDevice(&dev) == hipSuccess && release(dev);
   }
 
  private:

@@ -1113,7 +1113,7 @@ int persistent_create(Handle* h) {
     // (16384^2 x 1000 sweeps takes 0.08 seconds)
     cfg.timeout_s = 120.0;
     int rc = chm_init(0, nullptr, &cfg);
-    if (rc == CHM_E_NOMEM && DevCache::get().release())
+    if (rc == CHM_E_NOMEM && DevCache::get().release_current())
       rc = chm_init(0, nullptr, &cfg);
     if (rc != CHM_OK) return fail(rc, "chm_init: %s", chm_last_error());
   }
