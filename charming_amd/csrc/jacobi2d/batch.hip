@@ -1705,6 +1705,7 @@ struct Server {
   int mode = CHM_SERVE_ENGINE;
   Engine e;
   jac::DevBlock mem;
+  bool serving = false;  // the engine was announced to the kept memory
   char* pool = nullptr;  // mem's start
   size_t pool_size = 0;
   std::map<size_t, size_t> free_blocks;  // offset -> size
@@ -1837,6 +1838,7 @@ static void server_free(Server* s, bool idle) {
     s->worker.join();
   }
   plain_ctx_free(s->pc);
+  if (s->serving) jac::DevCache::get().serving(s->mem.dev, -1);
   idle = idle && s->worker_rc == CHM_OK;
   jac::DevCache::get().put(s->mem, idle);
   engine_free(s->e, idle);
@@ -1854,6 +1856,9 @@ extern "C" {
 
 int chm_jacobi2d_release_memory(void) {
   (void)jac::DevCache::get().release(jac::DevCache::kAllDevices);
+  if (jac::DevCache::get().held_back())
+    return fail(CHM_E_BUSY, "a server is running: its device's memory stays "
+                            "until it has stopped");
   return CHM_OK;
 }
 
@@ -2101,6 +2106,8 @@ int chm_jacobi2d_server_start(const chm_server_config* cfg, void** handle) {
     s->free_blocks[0] = budget;
     for (int i = (int)kMaxSlots - 1; i >= 0; i--) s->free_slots.push_back(i);
     if (s->mode == CHM_SERVE_ENGINE) {
+      jac::DevCache::get().serving(s->mem.dev, +1);
+      s->serving = true;
       rc = engine_launch(s->e);
     } else {
       int dev = 0;

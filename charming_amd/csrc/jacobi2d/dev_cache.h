@@ -107,7 +107,7 @@ class DevCache {
   }
 
   // Gives back what is kept on `dev` (kAllDevices: on any); false if nothing
-  // was.
+  // was.  Not where a server runs: see serving().
   bool release(int dev) {
     void* out[kBlocks];
     int n_out = 0;
@@ -115,12 +115,30 @@ class DevCache {
       std::lock_guard<std::mutex> lk(mu_);
       for (int i = n_ - 1; i >= 0; i--) {
         if (dev != kAllDevices && kept_[i].b.dev != dev) continue;
+        if (servers(kept_[i].b.dev) > 0) continue;
         out[n_out++] = kept_[i].b.p;
         kept_[i] = kept_[--n_];
       }
     }
     for (int i = 0; i < n_out; i++) (void)hipFree(out[i]);
     return n_out > 0;
+  }
+  // A server's engine starts (+1) or has stopped (-1) on `dev`.  hipFree waits
+  // for every kernel of the device, and this one ends only when its owner, who
+  // may be the thread that frees, stops it: what is kept goes back before it
+  // starts, and nothing while it runs (an allocation that fails then fails at
+  // once).
+  void serving(int dev, int change) {
+    if (change > 0) (void)release(dev);
+    std::lock_guard<std::mutex> lk(mu_);
+    if (dev >= 0 && dev < kDevices) servers_[dev] += change;
+  }
+  // Something is kept that a running server holds back.
+  bool held_back() {
+    std::lock_guard<std::mutex> lk(mu_);
+    for (int i = 0; i < n_; i++)
+      if (servers(kept_[i].b.dev) > 0) return true;
+    return false;
   }
   bool release_current() {
     int dev = 0;
@@ -130,12 +148,17 @@ class DevCache {
  private:
   using Clock = std::chrono::steady_clock;
   static constexpr int kBlocks = 48;
+  static constexpr int kDevices = 64;
   static constexpr int kKeepSeconds = 10;
   struct Kept {
     DevBlock b;
     Clock::time_point t;
   };
+  int servers(int dev) const {
+    return dev >= 0 && dev < kDevices ? servers_[dev] : 0;
+  }
   std::mutex mu_;
+  int servers_[kDevices] = {};
   Kept kept_[kBlocks];
   int n_ = 0;
 };

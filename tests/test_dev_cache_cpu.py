@@ -21,6 +21,7 @@ struct FakeHip {
   std::map<void*, std::pair<int, size_t>> blocks;
   char* next = (char*)4096;
   int frees = 0;
+  bool running[2] = {false, false};  // a kernel that this thread has to stop
 };
 inline FakeHip& fake() { static FakeHip* f = new FakeHip; return *f; }
 inline int& cur_dev() { static thread_local int d = 0; return d; }
@@ -47,6 +48,7 @@ inline hipError_t hipFree(void* p) {
   std::lock_guard<std::mutex> lk(f.mu);
   auto it = f.blocks.find(p);
   if (it == f.blocks.end()) abort();  // freed twice, or never taken
+  if (f.running[it->second.first]) abort();  // would wait for ever
   f.used[it->second.first] -= it->second.second;
   f.blocks.erase(it);
   f.frees++;
@@ -110,6 +112,28 @@ TESTS = {
     CHECK(fake().used[0] == 55 * MB);
     DevCache::get().put(take(20 * MB), false);  // work that failed: not kept
     CHECK(fake().used[0] == 55 * MB);""",
+    "server": r"""
+    // what is kept goes back before a server's engine starts; while it runs a
+    // failing allocation fails at once, and nothing is given back there
+    keep(0, 40 * MB);
+    keep(1, 50 * MB);
+    (void)hipSetDevice(0);
+    const DevBlock pool = take(700 * MB);
+    DevCache::get().serving(0, +1);
+    CHECK(fake().used[0] == 700 * MB && fake().used[1] == 50 * MB);
+    fake().running[0] = true;
+    keep(0, 60 * MB);  // another thread's batch ends meanwhile
+    void* p = nullptr;
+    CHECK(DevCache::get().alloc(&p, 90 * MB) == hipErrorOutOfMemory);
+    CHECK(DevCache::get().release(DevCache::kAllDevices));  // device 1's
+    CHECK(fake().used[0] == 760 * MB && fake().used[1] == 0);
+    CHECK(DevCache::get().held_back());
+    fake().running[0] = false;
+    DevCache::get().serving(0, -1);
+    DevCache::get().put(pool, true);
+    CHECK(!DevCache::get().held_back());
+    CHECK(DevCache::get().release(0));
+    CHECK(fake().used[0] == 0);""",
 }
 
 
