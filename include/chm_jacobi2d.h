@@ -216,9 +216,10 @@ int chm_jacobi2d_batch_run(const chm_batch_problem* probs, int n,
                            int* iters_done);
 
 /* Batches and servers keep the device memory they took for the next one, up
- * to an eighth of the device's.  It goes back here; when an allocation of
- * this library's solves, batches and servers on the same device fails; and
- * before a server's engine starts there.  While that engine runs nothing is
+ * to an eighth of the device's.  It goes back here; once it has not been used
+ * for ten seconds; when an allocation of this library's solves, batches and
+ * servers on the same device fails; and before a server's engine starts
+ * there.  While that engine runs nothing is
  * given back on its device (freeing waits for every kernel, and this one ends
  * only when the server is stopped): CHM_E_BUSY if something is kept there. */
 int chm_jacobi2d_release_memory(void);

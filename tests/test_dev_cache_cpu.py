@@ -12,8 +12,16 @@ HIP = r"""
 #pragma once
 #include <stddef.h>
 #include <stdlib.h>
+#include <atomic>
+#include <chrono>
 #include <map>
 #include <mutex>
+#include <thread>
+enum hipStreamCaptureMode { hipStreamCaptureModeGlobal, hipStreamCaptureModeRelaxed };
+inline hipStreamCaptureMode& capture_mode() {
+  static thread_local hipStreamCaptureMode m = hipStreamCaptureModeGlobal;
+  return m;
+}
 enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2 };
 struct FakeHip {
   std::mutex mu;
@@ -22,11 +30,17 @@ struct FakeHip {
   char* next = (char*)4096;
   int frees = 0;
   bool running[2] = {false, false};  // a kernel that this thread has to stop
+  bool capturing = false;            // a global capture is under way
+  std::atomic<int> free_ms{0};       // how long a free takes
 };
 inline FakeHip& fake() { static FakeHip* f = new FakeHip; return *f; }
 inline int& cur_dev() { static thread_local int d = 0; return d; }
 inline hipError_t hipGetDevice(int* d) { *d = cur_dev(); return hipSuccess; }
 inline hipError_t hipSetDevice(int d) { cur_dev() = d; return hipSuccess; }
+inline hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {
+  std::swap(*m, capture_mode());
+  return hipSuccess;
+}
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipDeviceTotalMem(size_t* t, int) {
   *t = fake().total;
@@ -45,10 +59,12 @@ hipError_t hipMalloc(T** p, size_t n) {
 }
 inline hipError_t hipFree(void* p) {
   FakeHip& f = fake();
+  std::this_thread::sleep_for(std::chrono::milliseconds(f.free_ms));
   std::lock_guard<std::mutex> lk(f.mu);
   auto it = f.blocks.find(p);
   if (it == f.blocks.end()) abort();  // freed twice, or never taken
   if (f.running[it->second.first]) abort();  // would wait for ever
+  if (f.capturing && capture_mode() != hipStreamCaptureModeRelaxed) abort();
   f.used[it->second.first] -= it->second.second;
   f.blocks.erase(it);
   f.frees++;
@@ -59,6 +75,7 @@ MAIN = r"""
 #include "dev_cache.h"
 #include <stdio.h>
 #include <string>
+#include <vector>
 using chm::jac::DevBlock;
 using chm::jac::DevCache;
 #define CHECK(x) \
@@ -68,6 +85,22 @@ static DevBlock take(size_t bytes) {
   DevBlock b;
   CHECK(DevCache::get().take(&b, bytes) == hipSuccess);
   return b;
+}
+static size_t used(int dev) {
+  std::lock_guard<std::mutex> lk(fake().mu);
+  return fake().used[dev];
+}
+static void set(bool& flag, bool v) {
+  std::lock_guard<std::mutex> lk(fake().mu);
+  flag = v;
+}
+static void sleep_ms(int ms) {
+  std::this_thread::sleep_for(std::chrono::milliseconds(ms));
+}
+// used(dev) == bytes within five seconds
+static bool comes_to(int dev, size_t bytes) {
+  for (int i = 0; i < 500 && used(dev) != bytes; i++) sleep_ms(10);
+  return used(dev) == bytes;
 }
 static void keep(int dev, size_t bytes) {
   (void)hipSetDevice(dev);
@@ -134,6 +167,102 @@ TESTS = {
     CHECK(!DevCache::get().held_back());
     CHECK(DevCache::get().release(0));
     CHECK(fake().used[0] == 0);""",
+    "timed": r"""
+    // what is not used for a while goes back by itself, also under another
+    // thread's graph capture, and again after all had gone
+    DevCache& c = *new DevCache(std::chrono::milliseconds(400));
+    for (int turn = 0; turn < 2; turn++) {
+      DevBlock a, b;
+      CHECK(c.take(&a, 30 * MB) == hipSuccess);
+      CHECK(c.take(&b, 50 * MB) == hipSuccess);
+      c.put(a, true);
+      sleep_ms(200);
+      set(fake().capturing, true);
+      c.put(b, true);
+      CHECK(used(0) == 80 * MB);
+      CHECK(comes_to(0, 50 * MB) && comes_to(0, 0));
+      set(fake().capturing, false);
+    }
+    // a block in use stays, one given to a new user too
+    DevBlock d, e;
+    CHECK(c.take(&d, 30 * MB) == hipSuccess);
+    c.put(d, true);
+    sleep_ms(200);
+    CHECK(c.take(&e, 30 * MB) == hipSuccess && e.p == d.p);
+    sleep_ms(600);
+    CHECK(used(0) == 30 * MB);
+    c.put(e, true);
+    CHECK(comes_to(0, 0));""",
+    "timed_server": r"""
+    // not while a server runs, whose start waits for frees under way
+    DevCache& c = *new DevCache(std::chrono::milliseconds(200));
+    DevBlock a, b;
+    CHECK(c.take(&a, 30 * MB) == hipSuccess);
+    c.put(a, true);
+    fake().free_ms = 300;
+    sleep_ms(350);  // (its free is under way, or about to be)
+    c.serving(0, +1);
+    CHECK(used(0) == 0);
+    set(fake().running[0], true);
+    CHECK(c.take(&b, 30 * MB) == hipSuccess);
+    c.put(b, true);
+    sleep_ms(700);
+    CHECK(used(0) == 30 * MB && c.held_back());
+    set(fake().running[0], false);
+    c.serving(0, -1);
+    CHECK(comes_to(0, 0));""",
+    "failing_meanwhile": r"""
+    // an allocation that fails while the thread frees waits for it
+    DevCache& c = *new DevCache(std::chrono::milliseconds(200));
+    DevBlock a;
+    CHECK(c.take(&a, 90 * MB) == hipSuccess);
+    c.put(a, true);
+    fake().free_ms = 400;
+    sleep_ms(400);
+    void* p = nullptr;
+    CHECK(c.alloc(&p, 790 * MB) == hipSuccess);""",
+    "stop": r"""
+    // the thread ends on request, at once, and nothing is kept or freed by it
+    // afterwards
+    DevCache& c = *new DevCache(std::chrono::milliseconds(300));
+    DevBlock a, b;
+    CHECK(c.take(&a, 30 * MB) == hipSuccess);
+    CHECK(c.take(&b, 20 * MB) == hipSuccess);
+    c.put(a, true);
+    const auto t0 = std::chrono::steady_clock::now();
+    c.stop();
+    CHECK(std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(250));
+    c.put(b, true);
+    CHECK(used(0) == 30 * MB);
+    sleep_ms(500);
+    CHECK(used(0) == 30 * MB);""",
+    "threads": r"""
+    // takes and returns by several threads beside the one that gives back
+    DevCache& c = *new DevCache(std::chrono::milliseconds(3));
+    std::vector<std::thread> ts;
+    for (int t = 0; t < 6; t++)
+      ts.emplace_back([&c, t] {
+        (void)hipSetDevice(t & 1);
+        for (int i = 0; i < 400; i++) {
+          DevBlock a, b;
+          CHECK(c.take(&a, (1 + (i * 7 + t) % 9) * MB) == hipSuccess);
+          CHECK(c.take(&b, (1 + (i * 5 + t) % 30) * MB) == hipSuccess);
+          CHECK(a.p != b.p);
+          if (i % 40 == t) sleep_ms(5);
+          c.put(a, true);
+          c.put(b, i % 3 != 0);
+          if (i % 50 == t) c.release(t & 1);
+          if (i % 60 == t) {
+            c.serving(t & 1, +1);
+            c.serving(t & 1, -1);
+          }
+        }
+      });
+    for (auto& t : ts) t.join();
+    CHECK(comes_to(0, 0) && comes_to(1, 0));""",
+    "exit": r"""
+    // a process may end with memory kept and its thread waiting
+    keep(0, 40 * MB);""",
 }
 
 

@@ -1,6 +1,7 @@
-"""Kept device memory beside a running server: giving memory back waits for
-every kernel of the device, and a server's engine ends only when its owner
-stops it, so nothing may be given back while it runs."""
+"""When kept device memory goes back: before a server's engine starts and not
+while it runs (giving memory back waits for every kernel of the device, and
+that engine ends only when its owner stops it), and by itself once it has not
+been used for a while."""
 import threading
 import time
 
@@ -39,3 +40,28 @@ def test_release_beside_a_server_returns():
         guard.cancel()
         srv.stop()
     cam.release_memory()
+
+
+def test_unused_memory_goes_back_by_itself():
+    # after ten seconds, here while another thread captures a graph, which
+    # the free must not end
+    import charming_amd as cam
+    probs = [dict(width=1500, height=1400, iters=20, seed=i) for i in range(9)]
+    arena = 9 * 3 * 1500 * 1400 * 8
+    want = cam.batch_run(probs)["hashes"]
+    cam.release_memory()
+    x = torch.zeros(1000, device="cuda")
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    assert cam.batch_run(probs)["hashes"] == want
+    assert before - torch.cuda.mem_get_info()[0] >= arena
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x.add_(1)
+        time.sleep(13)
+    for k in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool((x == k + 1).all())
+    assert before - torch.cuda.mem_get_info()[0] < arena
+    assert cam.batch_run(probs)["hashes"] == want
