@@ -1565,7 +1565,7 @@ struct PlainCtx {
 
 static int plain_ctx_init(PlainCtx& c) {
   CHM_TRY_HIP(hipStreamCreateWithFlags(&c.s, hipStreamNonBlocking));
-  CHM_TRY_HIP(hipMalloc(&c.d_words, 64));
+  CHM_TRY_HIP(jac::DevCache::get().alloc(&c.d_words, 64));
   CHM_TRY(host_alloc((void**)&c.h_words, 128));
   for (auto& e : c.ev)
     CHM_TRY_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));

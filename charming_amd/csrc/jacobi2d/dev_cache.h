@@ -139,6 +139,14 @@ class DevCache {
     if (dev >= 0 && dev < kDevices) servers_[dev] += change;
     if (change > 0) idle_.wait(lk, [this] { return !freeing_; });
   }
+  // Bytes that are kept on `dev` and an allocation here could have.
+  size_t available(int dev) {
+    std::lock_guard<std::mutex> lk(mu_);
+    size_t sum = 0;
+    for (int i = 0; i < n_; i++)
+      if (kept_[i].b.dev == dev && servers(dev) == 0) sum += kept_[i].b.bytes;
+    return sum;
+  }
   // Something is kept that a running server holds back.
   bool held_back() {
     std::lock_guard<std::mutex> lk(mu_);

@@ -776,7 +776,10 @@ int chm_jacobi2d_chare_phases(void* handle, double* out, size_t out_elems,
 
 int chm_device_memory(size_t* free_bytes, size_t* total_bytes) {
   if (!free_bytes || !total_bytes) return fail(CHM_E_INVALID, "null argument");
+  int dev = 0;
+  CHM_TRY_HIP(hipGetDevice(&dev));
   CHM_TRY_HIP(hipMemGetInfo(free_bytes, total_bytes));
+  *free_bytes += DevCache::get().available(dev);
   return CHM_OK;
 }
 

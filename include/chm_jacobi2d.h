@@ -156,7 +156,8 @@ const char* chm_jacobi2d_last_error(void);
 int chm_hbm_copy_probe(size_t bytes, int reps, double* ms_per_copy);
 
 /* Free and total HBM of the current device, in bytes (what an admission
- * budget can be sized from).  No reference counterpart. */
+ * budget can be sized from: memory kept for the next batch or server counts
+ * as free).  No reference counterpart. */
 int chm_device_memory(size_t* free_bytes, size_t* total_bytes);
 
 /* Sanity hook with no GPU work: returns the ABI version. */

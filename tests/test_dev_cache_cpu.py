@@ -160,13 +160,26 @@ TESTS = {
     CHECK(DevCache::get().alloc(&p, 90 * MB) == hipErrorOutOfMemory);
     CHECK(DevCache::get().release(DevCache::kAllDevices));  // device 1's
     CHECK(fake().used[0] == 760 * MB && fake().used[1] == 0);
-    CHECK(DevCache::get().held_back());
+    CHECK(DevCache::get().held_back() && DevCache::get().available(0) == 0);
     fake().running[0] = false;
     DevCache::get().serving(0, -1);
     DevCache::get().put(pool, true);
     CHECK(!DevCache::get().held_back());
     CHECK(DevCache::get().release(0));
     CHECK(fake().used[0] == 0);""",
+    "available": r"""
+    // what an allocation could have on a device counts as free there
+    keep(0, 40 * MB);
+    keep(0, 30 * MB);
+    keep(1, 20 * MB);
+    CHECK(DevCache::get().available(0) == 70 * MB);
+    CHECK(DevCache::get().available(1) == 20 * MB);
+    (void)hipSetDevice(0);
+    const DevBlock b = take(40 * MB);
+    CHECK(DevCache::get().available(0) == 30 * MB);
+    void* p = nullptr;
+    CHECK(DevCache::get().alloc(&p, 760 * MB) == hipSuccess);
+    CHECK(DevCache::get().available(0) == 0);""",
     "timed": r"""
     // what is not used for a while goes back by itself, also under another
     // thread's graph capture, and again after all had gone

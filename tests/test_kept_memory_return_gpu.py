@@ -65,3 +65,18 @@ def test_unused_memory_goes_back_by_itself():
         assert bool((x == k + 1).all())
     assert before - torch.cuda.mem_get_info()[0] < arena
     assert cam.batch_run(probs)["hashes"] == want
+
+
+def test_kept_memory_counts_as_free():
+    # a budget sized from the free memory is the same before and after a batch
+    import charming_amd as cam
+    probs = [dict(width=1500, height=1400, iters=20, seed=i) for i in range(9)]
+    arena = 9 * 3 * 1500 * 1400 * 8
+    cam.batch_run(probs)
+    cam.release_memory()
+    before = cam.device_memory()
+    cam.batch_run(probs)
+    after = cam.device_memory()
+    assert before[1] == after[1] and abs(after[0] - before[0]) < arena // 2
+    assert torch.cuda.mem_get_info()[0] <= after[0] - arena
+    cam.release_memory()
