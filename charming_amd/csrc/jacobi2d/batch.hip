@@ -31,6 +31,7 @@
 #include "engine_dev.h"
 #include "jacobi2d_internal.h"
 #include "pipeline.h"
+#include "stop_filter.h"
 
 namespace chm {
 namespace eng {
@@ -413,31 +414,17 @@ __device__ inline bool pipe_tiles(const Request& r) {
   return (r.bs & 1) == 0 || r.tc == 1;
 }
 
-// Thread 0: the same for a filtered round run as groups of waves, which sums
-// the last sweep only.  With D_j = u_j - u_{j-1}, D_{j+1} = 0.2 A D_j + e:
-// A (a cell and its four neighbours) is symmetric with norm at most 5, and e
-// is what two sweeps round, at most 2 x 3.8 x 2^-53 M a cell, M the largest
-// |u|.  So |D_j| >= |D_n| - n E over the N cells for every earlier sweep,
-// E = sqrt(N) 2^-48 M holding e four times over (0.2 is rounded up, which
-// grows |u| and |D_j| by 2^-53 a sweep), and one sum of two operations per
-// cell and round replaces n of three.  With it the exact S_j, which truncates
-// less than 1 a cell as above, exceeds 2^56 (|D_n| - n E)^2 - N.
+// Thread 0: whether a filtered round that ran as groups of waves, which sum
+// the last sweep only, may hold the stop.
 __device__ bool pipe_may_stop(Prob& p, const Request& r, int sk) {
-  const double thr = r.tol2 * u128d(ald(&p.s0[0]), ald(&p.s0[1]));
-  if (!(thr < 0x1.0p62)) return true;
-  const double n = (double)r.W * (double)r.H;
-  const double a =
-      __longlong_as_double((long long)ald((uint64_t*)&p.resd[sk][0]));
-  const double m = r.init_mode == CHM_INIT_REFERENCE
-                       ? 10.0
-                       : fmax(1.0, fabs(r.boundary));
-  const double x = sqrt(a) * (1.0 - 0x1.0p-20) -
-                   (double)r.depth * sqrt(n) * m * 0x1.0p-48;
-  return !(x > 0.0 &&
-           x * x * 0x1.0p56 * (1.0 - 0x1.0p-20) - n > thr * (1.0 + 0x1.0p-20));
+  return jac::last_sum_may_stop(
+      r.tol2 * u128d(ald(&p.s0[0]), ald(&p.s0[1])),
+      __longlong_as_double((long long)ald((uint64_t*)&p.resd[sk][0])),
+      (double)r.W * (double)r.H, (double)r.depth,
+      r.init_mode == CHM_INIT_REFERENCE ? 10.0 : fmax(1.0, fabs(r.boundary)));
 }
 
-// Thread 0: whether a filtered round may hold the stop.  The exact residual
+// Thread 0: the same for one that summed every sweep.  The exact residual
 // of sweep j is S_j = sum floor(fl(d^2) 2^56) over the cells (saturating at
 // 2^64 - 1), so S_j >= 2^56 T_j - N with T_j = sum fl(d^2) when no term
 // saturates, and the FP64 sum A_j of the same fl(d^2) (N <= 2^30 terms, any
