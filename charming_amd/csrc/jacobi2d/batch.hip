@@ -1956,7 +1956,7 @@ int chm_jacobi2d_batch_autotune(const chm_batch_problem* probs, int n,
   // pick ran 102.6-103.2 ms, the 32-sweep samples' pick 114-122 ms.)
   const int cap = sample_iters > 0 ? (sample_iters + 15) / 16 * 16 : 0;
   // tile sides tried per size class: the powers of two and the multiples
-  // of the deep pass's window (112 columns at eight sweeps, 96 at sixteen)
+  // of the window pass's window (112 columns at eight sweeps, 96 at sixteen)
   static const int kBlocks8[] = {64, 112, 128, 224, 256, 448, 512};
   static const int kBlocks16[] = {64, 96, 128, 192, 256, 384, 512};
   // and for groups of waves, what their windows give
@@ -2016,17 +2016,18 @@ int chm_jacobi2d_batch_autotune(const chm_batch_problem* probs, int n,
   if (top < 0) return fail(CHM_E_DEVICE, "no autotune candidate ran");
   std::vector<int> blocks = rule_blocks(top_cfg.wg_threads);
   const bool wide = deep_for_threads(top_cfg.wg_threads) == kDeepWide;
-  const int* kBlocks = top_cfg.wg_threads == kPipeThreads ? kBlocksPipe
-                       : wide                             ? kBlocks16
-                                                          : kBlocks8;
-  const int n_blocks = wide ? (int)(sizeof(kBlocks16) / sizeof(int))
-                            : (int)(sizeof(kBlocks8) / sizeof(int));
+  const std::vector<int> sides(
+      top_cfg.wg_threads == kPipeThreads ? std::begin(kBlocksPipe)
+      : wide                             ? std::begin(kBlocks16)
+                                         : std::begin(kBlocks8),
+      top_cfg.wg_threads == kPipeThreads ? std::end(kBlocksPipe)
+      : wide                             ? std::end(kBlocks16)
+                                         : std::end(kBlocks8));
   // 2. tile side per size class, one class at a time (largest first)
   for (int c = n_cls - 1; c >= 0; c--) {
     std::vector<int> trial = blocks;
     int best_b = -1;
-    for (int bi = 0; bi < n_blocks; bi++) {
-      const int b = kBlocks[bi];
+    for (const int b : sides) {
       bool any = false;
       for (int i = 0; i < n; i++)
         if (cls[i] == c) {
