@@ -292,7 +292,8 @@ def batch_run(probs, wg_threads=0, block=0, panel_chunks=0, rows_in_flight=0,
 
 def release_memory():
     """Give back the device memory that batches and servers keep between
-    calls (at most an eighth of the device's)."""
+    calls (at most an eighth of the device's, for ten seconds unused).  BUSY
+    if something is kept on a device whose server is running."""
     _check(jacobi_lib().chm_jacobi2d_release_memory())
 
 

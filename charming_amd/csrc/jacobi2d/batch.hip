@@ -225,9 +225,10 @@ __device__ __noinline__ void do_round_deep(const double* in, double* out,
 }
 
 // 4 NST sweeps of a tile by groups of four waves (pipeline.h).  SUM: the
-// FP64 sum of the last sweep's squared changes is added to *sum.  A 544 x 544
-// tile takes sixteen sweeps in 0.28 ms on a busy card, about 0.45 with
-// do_round_deep.
+// FP64 sum of the last sweep's squared changes is added to *sum.  With every
+// CU busy (1024 problems of one tile) a round of a 544 x 544 tile takes 440 us
+// with its task's fences, 780 with do_round_deep; of 288 x 288 169 against
+// 272, of 160 x 160 88 against 132, of 96 x 96 68 against 82.
 template <int T, int NST, bool SUM>
 __device__ __noinline__ void do_round_pipe(const Request* rp, int r0, int r1,
                                            int c0, int c1, int src, int dst,
@@ -1055,7 +1056,10 @@ static double now_s() {
 
 // Tile sides of engines whose rounds run as groups of waves, what a window of
 // 3, 5 or 9 columns per lane gives after sixteen sweeps (and half of the
-// first, for little work), and the time of a tile's round in us.
+// first, for little work), and the time of a tile's round in us on a card with
+// little else to do.  The rules below compare such times with each other, so
+// that their ratios count: 5.7 : 2.4 : 1.3 : 1 with a task's 8 us; with every
+// CU busy the rounds take 440, 169, 88 and 68 us, 6.4 : 2.5 : 1.3 : 1.
 constexpr int kPipeSides[] = {544, 288, 160, 96};
 constexpr double kPipeTimes[] = {300, 120, 61, 46};
 constexpr int kPipeSideN = 4;
@@ -1083,10 +1087,10 @@ static int pick_block(int W, int H, int block, int deep) {
 }
 
 // Tile sides of a batch for an engine of groups of waves (blocks[i], those
-// not given already): the largest side costs least per cell (1.0 ns a cell
-// and round at 544, 1.5 at 288, 2.5 at 160, 5.2 at 96), but a problem's
-// rounds follow each other, so the one whose rounds take longest is cut
-// finer while that is longer than the whole batch's work spread over the
+// not given already): the largest side costs least per cell (on a busy card
+// 1.5 ns a cell and round at 544, 2.0 at 288, 3.4 at 160, 7.4 at 96), but a
+// problem's rounds follow each other, so the one whose rounds take longest is
+// cut finer while that is longer than the whole batch's work spread over the
 // workgroups.
 static void pick_blocks(const chm_batch_problem* probs, int n, int n_wg,
                         std::vector<int>& blocks) {
@@ -1736,9 +1740,10 @@ static int serve_block(int W, int H, int n_wg, int resident, int ow) {
 }
 
 // The same for engines of groups of waves, of their sides: a finer one where
-// it at least halves the round on this request's share of the workgroups (it
-// costs 1.5 to 2 times as much per cell, which requests that arrive beside
-// this one would miss: the burst of 24 requests of 256..8192 per side).
+// it at least halves the round on this request's share of the workgroups.  It
+// costs 1.4 to 2.1 times as much per cell, which requests that arrive beside
+// this one would miss.  (The factor of two was set on one workload, a burst of
+// 24 requests of 256..8192 per side, and others were not tried.)
 static int serve_block_pipe(int W, int H, int n_wg, int resident) {
   const int64_t share = std::max<int64_t>(1, n_wg / (1 + resident));
   int best = kPipeSides[0];

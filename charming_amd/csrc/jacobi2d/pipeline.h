@@ -444,7 +444,7 @@ __device__ __noinline__ void pipe_wave(int role, int lds_off) {
   // places.  The wave's first half of a step runs at a higher priority:
   // two waves share a SIMD, and with equal priorities the older one took
   // all the issue slots it could, its group ran ahead and the other group
-  // finished alone (1.20 -> 1.11 ms per sixteen sweeps of 1024 x 1024).
+  // finished alone (1.20 -> 1.13-1.17 ms per sixteen sweeps of 1024 x 1024).
   auto step = [&](int u, int n) __attribute__((always_inline)) {
     const int e = (NS - u) % NS;
     __builtin_amdgcn_s_setprio(1);
@@ -571,9 +571,11 @@ __device__ __noinline__ void pipe_wave(int role, int lds_off) {
       for (int j = 0; j < K; j++) row_w[j] = O[j];
     }
   };
-  // sweep s of step n makes row q0 + n - s: the turns up to tA may meet the
-  // top ring row, later ones the bottom one (a block is at least 2 NS rows
-  // away from meeting both in one turn: its D rows above and below)
+  // sweep s of step n makes row q0 + n - s: the turns that begin before tA may
+  // meet the top ring row, later ones the bottom one.  The last of the former
+  // ends with row top + NST + NS - 2 = top + 2 NST at most: the bottom ring row
+  // lies beyond it in a grid of D = 4 NST rows or more.
+  static_assert(D + 1 > NST + NS - 2, "both ring rows in one turn");
   const int tA = top != kNoRing ? top - q0 + NST : 0;
   for (int t0 = 0; t0 < n_steps; t0 += NS) {
     ring_row = t0 < tA ? top : bottom;
@@ -616,7 +618,8 @@ __device__ __forceinline__ void pipe_group(int cols, int role, int off) {
 // A block of an array: output columns [cols.c0, cols.c1) and rows [r0, r1),
 // the grid's ring rows and columns (kNoRing where they are out of reach) and
 // the part of the input that may be read (odd columns to lo_col at least).
-// Ring rows, if both are in reach, are sixteen rows apart or more.
+// Ring rows, if both are in reach, are more than 2 NST rows apart (callers'
+// grids have 4 NST rows at least).
 struct PipeBlock {
   const double* in;
   double* out;
@@ -637,7 +640,6 @@ __device__ inline PipeLds* pipe_lds() {
 // Workgroup-collective (T threads, all waves): 4 NST fused sweeps of the
 // block.  Groups take whole windows in turn; of an odd number the last one
 // is halved by rows (so both groups always have as many windows to do).
-// lds: one PipeLds per group of four waves.
 template <int T, int NST, bool SUM>
 __device__ __forceinline__ void pipe_block(const PipeBlock& b, double* sum) {
   constexpr int G = T / 64 / kPipeWaves;

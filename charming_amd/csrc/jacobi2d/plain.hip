@@ -439,7 +439,7 @@ __global__ void end_noalloc_kernel(const double* g, double* copy, int W, int H,
 // bands: 1021 x 683 x 100 took 5.28 ms, now 0.21; 2800 x 2800 x 200 16.3 ms,
 // now 1.04 (5 TB/s of the caches would allow 0.3; the tiles' margins and the
 // filling of their pipelines double the arithmetic); 64 x 64 x 10 345 us,
-// now 34, in five launches.
+// now 34, in six launches.
 constexpr int kPassThreads = 512;
 template <int NST>
 __global__ void __launch_bounds__(kPassThreads)

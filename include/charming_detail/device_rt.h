@@ -832,7 +832,8 @@ __device__ __noinline__ void pe_loop() {
   while (pe_step()) {
     // (a request is made before the turn's last barrier.  Tested here, not in
     // run_work, whose entry parks some 190 registers of every lane: called
-    // after each message, it made that 10 us of the 12 that a message took.)
+    // after each message, it made that 10 us of the 12 that a message of a
+    // program with a work hook took.)
     if (lds().has_work) run_work();
     __syncthreads();
   }

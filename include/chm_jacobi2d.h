@@ -66,7 +66,9 @@ typedef struct chm_jacobi_tuning {
   int band_rows;     /* rows per wave band (plain form; persistent form with
                         halos 3+ deep: < 0 = one contiguous share of the
                         chare per wave, 0 = 256 for chares of 1024+ rows,
-                        else contiguous shares) */
+                        else contiguous shares; with 0, rounds of sixteen
+                        sweeps but the last run whole columns of the chare
+                        by groups of waves instead) */
   int wg_waves;      /* waves per workgroup (plain form) */
   int overlap;       /* persistent form: 1 = sweep the edges first and send the
                         halos before the interior (default 0; depth 1 only) */
@@ -167,10 +169,11 @@ int chm_jacobi2d_abi_version(void);
  * Batched and served forms.  No reference counterpart: the reference runs
  * one Jacobi2D problem per job (examples/jacobi2d/jacobi2d.cu:26-77).  Here
  * many independent problems share one persistent launch of a task engine:
- * each problem is cut into square chare tiles, one task is one round (two
- * fused sweeps) of one tile, a tile's completion is the (zero-copy) halo
- * message that releases its neighbours, and idle workgroups steal ready
- * tasks from the others.
+ * each problem is cut into square chare tiles, one task is one round of one
+ * tile (sixteen or eight fused sweeps, twelve or six with a tolerance, two of
+ * thin grids), a tile's completion is the (zero-copy) halo message that
+ * releases its neighbours, and idle workgroups steal ready tasks from the
+ * others.
  * Every problem's result is bit-identical to the same problem solved alone
  * (and to the monolithic CPU sweep).
  * ------------------------------------------------------------------------ */
@@ -192,7 +195,8 @@ typedef struct chm_batch_config {
                          workgroups per CU, as many as stay resident; fixed
                          sweep counts go in rounds of sixteen fused sweeps
                          at 512 threads or fewer, of eight at 1024 */
-  int block;          /* tile side for problems with block 0 (0 = by size) */
+  int block;          /* tile side for problems with block 0 (0 = by size,
+                         at 512 threads by the batch's load) */
   int panel_chunks;   /* sweep shape: 1 or 2 (0 = 1) */
   int rows_in_flight; /* sweep shape: 2 or 4 (0 = 2) */
   double timeout_s;   /* watchdog (0 = 120 s) */
@@ -235,11 +239,11 @@ int chm_jacobi2d_batch_plain(const chm_batch_problem* probs, int n,
 
 /* Autotuner: picks the workgroup size and sweep shape, and a tile side per
  * problem (blocks_out[i]) from {64, 96, 128, 192, 256, 384, 512} for
- * workgroups of 512 threads or fewer, {64, 112, 128, 224, 256, 448, 512}
- * for 1024, by coordinate descent over size classes, timing short engine
- * runs of the whole batch with every problem capped at sample_iters sweeps
- * rounded up to a multiple of 16 (0 = no cap: full-length runs).  best_rate
- * = cell updates per second of the best. */
+ * workgroups of 256 threads, {96, 160, 192, 288, 384, 512, 544} for 512,
+ * {64, 112, 128, 224, 256, 448, 512} for 1024, by coordinate descent over
+ * size classes, timing engine runs of the whole batch with every problem
+ * capped at sample_iters sweeps rounded up to a multiple of 16 (0 = no cap:
+ * full-length runs).  best_rate = cell updates per second of the best. */
 int chm_jacobi2d_batch_autotune(const chm_batch_problem* probs, int n,
                                 int sample_iters, chm_batch_config* best,
                                 int* blocks_out, double* best_rate);
@@ -255,8 +259,9 @@ typedef struct chm_server_config {
   int max_active;      /* requests resident at once (0 = 4096) */
   int wg_threads, block, panel_chunks, rows_in_flight; /* as chm_batch_config
                           (wg_threads 0 = 512: tolerance rounds of twelve);
-                          block 0 = by load: a request gets about
-                          workgroups / (1 + resident requests) tiles */
+                          block 0 = by load: tiles as large as a request's
+                          share of the workgroups, 1 / (1 + resident
+                          requests), allows */
 } chm_server_config;
 
 typedef struct chm_server_completion {
@@ -275,8 +280,9 @@ typedef struct chm_server_stats {
   long long submitted, completed;
 } chm_server_stats;
 
-/* Start a server: allocates the grid pool (budget) once, launches the engine
- * (mode ENGINE) or a host worker thread (mode PLAIN). */
+/* Start a server: takes the grid pool (budget) once, new or kept from an
+ * earlier one, launches the engine (mode ENGINE) or a host worker thread
+ * (mode PLAIN). */
 int chm_jacobi2d_server_start(const chm_server_config* cfg, void** server);
 
 /* Admit one request: CHM_OK and *ticket, or CHM_E_BUSY when its grids do not
@@ -293,7 +299,8 @@ int chm_jacobi2d_server_poll(void* server, chm_server_completion* out,
 int chm_jacobi2d_server_stats(void* server, chm_server_stats* out);
 
 /* Wait for every admitted request to complete (up to timeout_s), then stop
- * the engine and free the pool.  abort_now = 1 stops at once. */
+ * the engine and give up the pool (kept for the next server or freed, see
+ * chm_jacobi2d_release_memory).  abort_now = 1 stops at once. */
 int chm_jacobi2d_server_stop(void* server, int abort_now, double timeout_s);
 
 #ifdef __cplusplus
