@@ -32,6 +32,7 @@
 #include "jacobi2d_internal.h"
 #include "pipeline.h"
 #include "stop_filter.h"
+#include "tile_rules.h"
 
 namespace chm {
 namespace eng {
@@ -1054,24 +1055,6 @@ static double now_s() {
   return ts.tv_sec + ts.tv_nsec * 1e-9;
 }
 
-// Tile sides of engines whose rounds run as groups of waves, what a window of
-// 3, 5 or 9 columns per lane gives after sixteen sweeps (and half of the
-// first, for little work), and the time of a tile's round in us on a card with
-// little else to do.  The rules below compare such times with each other, so
-// that their ratios count: 5.7 : 2.4 : 1.3 : 1 with a task's 8 us; with every
-// CU busy the rounds take 440, 169, 88 and 68 us, 6.4 : 2.5 : 1.3 : 1.
-constexpr int kPipeSides[] = {544, 288, 160, 96};
-constexpr double kPipeTimes[] = {300, 120, 61, 46};
-constexpr int kPipeSideN = 4;
-
-// A round of a tile of level l in us, of a problem `height` rows high (a
-// partial tile takes its share of the steps; a task costs about 8 us besides).
-static double pipe_tile_us(int height, int l) {
-  const int side = kPipeSides[l];
-  const double h = std::min(height, side);
-  return kPipeTimes[l] * (h / 2 + 38) / (side / 2 + 38) + 8;
-}
-
 // Tile side for a problem: `block` (> 0), or a rule that keeps tiles large
 // enough to amortise a task's fences and small enough to spread the problem,
 // in multiples of the window pass's window: 112 columns at eight sweeps
@@ -1084,59 +1067,6 @@ static int pick_block(int W, int H, int block, int deep) {
   if (side <= 256) return ow;
   if (side <= 1024) return 2 * ow;
   return 4 * ow;
-}
-
-// Tile sides of a batch for an engine of groups of waves (blocks[i], those
-// not given already): the largest side costs least per cell (on a busy card
-// 1.5 ns a cell and round at 544, 2.0 at 288, 3.4 at 160, 7.4 at 96), but a
-// problem's rounds follow each other, so the one whose rounds take longest is
-// cut finer while that is longer than the whole batch's work spread over the
-// workgroups.
-static void pick_blocks(const chm_batch_problem* probs, int n, int n_wg,
-                        std::vector<int>& blocks) {
-  struct Item {
-    double latency;
-    int i, level;
-    bool operator<(const Item& o) const { return latency < o.latency; }
-  };
-  auto rounds = [&](int i) { return (double)((probs[i].iters + 15) / 16); };
-  auto tiles = [&](int i, int side) {
-    return (double)((probs[i].width + side - 1) / side) *
-           ((probs[i].height + side - 1) / side);
-  };
-  auto tile_us = [&](int i, int l) { return pipe_tile_us(probs[i].height, l); };
-  double work = 0;  // us over all workgroups
-  std::vector<Item> heap;
-  for (int i = 0; i < n; i++) {
-    if (blocks[i] > 0) {
-      work += rounds(i) * tiles(i, blocks[i]) * 60;
-      continue;
-    }
-    int l = 0;  // no side beyond the next one that holds the problem
-    const int side = std::max(probs[i].width, probs[i].height);
-    while (l + 1 < kPipeSideN && side <= kPipeSides[l + 1]) l++;
-    blocks[i] = kPipeSides[l];
-    work += rounds(i) * tiles(i, kPipeSides[l]) * tile_us(i, l);
-    heap.push_back({rounds(i) * tile_us(i, l), i, l});
-  }
-  std::make_heap(heap.begin(), heap.end());
-  while (!heap.empty() && heap.front().latency > work / n_wg) {
-    std::pop_heap(heap.begin(), heap.end());
-    Item t = heap.back();
-    heap.pop_back();
-    if (t.level + 1 >= kPipeSideN ||
-        tiles(t.i, kPipeSides[t.level + 1]) >= (double)kMaxTiles)
-      break;  // cannot get shorter
-    const double was = rounds(t.i) * tiles(t.i, kPipeSides[t.level]) *
-                       tile_us(t.i, t.level);
-    t.level++;
-    blocks[t.i] = kPipeSides[t.level];
-    work += rounds(t.i) * tiles(t.i, kPipeSides[t.level]) *
-                tile_us(t.i, t.level) - was;
-    t.latency = rounds(t.i) * tile_us(t.i, t.level);
-    heap.push_back(t);
-    std::push_heap(heap.begin(), heap.end());
-  }
 }
 
 struct Built {
@@ -1451,7 +1381,7 @@ static int pipe_blocks(const chm_batch_problem* probs, int n,
     if (p.width < 1 || p.height < 1 || p.iters < 1) return CHM_OK;
     if (p.block > 0) sides[i] = p.block;
   }
-  pick_blocks(probs, n, cus, sides);
+  pick_blocks(probs, n, cus, kMaxTiles, sides);
   return CHM_OK;
 }
 
@@ -1737,29 +1667,6 @@ static int serve_block(int W, int H, int n_wg, int resident, int ow) {
     if (tiles >= target) return bs;
   }
   return 64;
-}
-
-// The same for engines of groups of waves, of their sides: a finer one where
-// it at least halves the round on this request's share of the workgroups.  It
-// costs 1.4 to 2.1 times as much per cell, which requests that arrive beside
-// this one would miss.  (The factor of two was set on one workload, a burst of
-// 24 requests of 256..8192 per side, and others were not tried.)
-static int serve_block_pipe(int W, int H, int n_wg, int resident) {
-  const int64_t share = std::max<int64_t>(1, n_wg / (1 + resident));
-  int best = kPipeSides[0];
-  double t_best = 0;
-  for (int l = 0; l < kPipeSideN; l++) {
-    const int bs = kPipeSides[l];
-    const int64_t tiles = (int64_t)((W + bs - 1) / bs) * ((H + bs - 1) / bs);
-    if (l > 0 && tiles >= (int64_t)kMaxTiles) break;
-    const double t =
-        (double)((tiles + share - 1) / share) * pipe_tile_us(H, l);
-    if (l == 0 || 2 * t <= t_best) {
-      best = bs;
-      t_best = t;
-    }
-  }
-  return best;
 }
 
 static bool pool_alloc(Server& s, size_t bytes, size_t* off) {
@@ -2130,7 +2037,7 @@ int chm_jacobi2d_server_submit(void* handle, const chm_batch_problem* pb,
   if (engine && pb->block <= 0 && block <= 0)
     block = s->e.threads == kPipeThreads
                 ? serve_block_pipe(pb->width, pb->height, s->e.d.n_wg,
-                                   (int)s->live.size())
+                                   (int)s->live.size(), kMaxTiles)
                 : serve_block(pb->width, pb->height, s->e.d.n_wg,
                               (int)s->live.size(),
                               jac::window_out_cols(
