@@ -1635,8 +1635,11 @@ struct Server {
     size_t off, bytes;
     uint32_t slot;
     double t_submit;
+    int64_t tiles;
+    double round_us;  // see ServeLoad
   };
   std::map<uint64_t, Live> live;  // ticket -> allocation
+  ServeLoad load;                 // of live
   uint64_t next_ticket = 0;
   uint64_t seen = 0;  // completion records consumed (engine ring)
   long long completed = 0;
@@ -2036,8 +2039,8 @@ int chm_jacobi2d_server_submit(void* handle, const chm_batch_problem* pb,
   int block = s->block;
   if (engine && pb->block <= 0 && block <= 0)
     block = s->e.threads == kPipeThreads
-                ? serve_block_pipe(pb->width, pb->height, s->e.d.n_wg,
-                                   (int)s->live.size(), kMaxTiles)
+                ? serve_block_pipe(pb->width, pb->height, s->e.d.n_wg, s->load,
+                                   kMaxTiles)
                 : serve_block(pb->width, pb->height, s->e.d.n_wg,
                               (int)s->live.size(),
                               jac::window_out_cols(
@@ -2065,7 +2068,13 @@ int chm_jacobi2d_server_submit(void* handle, const chm_batch_problem* pb,
   r.ticket = s->next_ticket++;
   r.slot = s->free_slots.back();
   s->free_slots.pop_back();
-  s->live[r.ticket] = Server::Live{off, bytes, r.slot, now_s()};
+  const int64_t tiles = (int64_t)r.tr * r.tc;
+  const Server::Live& l = s->live[r.ticket] =
+      Server::Live{off,     bytes, r.slot,
+                   now_s(), tiles, serve_round_us(r.H, tiles, r.bs)};
+  s->load.requests++;
+  s->load.tiles += l.tiles;
+  s->load.us += l.round_us;
   if (engine) {
     s->e.h_reqs[r.ticket & (s->e.d.req_cap - 1)] = r;
     __atomic_store_n(s->e.h_tail, r.ticket + 1, __ATOMIC_SEQ_CST);
@@ -2123,7 +2132,11 @@ int chm_jacobi2d_server_poll(void* handle, chm_server_completion* out,
     if (it != s->live.end()) {
       pool_free(*s, it->second.off, it->second.bytes);
       s->free_slots.push_back(it->second.slot);
+      s->load.requests--;
+      s->load.tiles -= it->second.tiles;
+      s->load.us -= it->second.round_us;
       s->live.erase(it);
+      if (s->live.empty()) s->load = ServeLoad();  // (no rounding is carried)
     }
     s->completed++;
   }

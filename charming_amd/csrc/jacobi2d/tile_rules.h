@@ -12,21 +12,25 @@
 namespace chm {
 namespace eng {
 
-// A side, and the time of a tile's round in us on a card with little else to
-// do.  The rules below compare such times with each other, so that their
-// ratios count: 5.7 : 2.4 : 1.3 : 1 with a task's 8 us; with every CU busy the
-// rounds take 440, 169, 88 and 68 us, 6.4 : 2.5 : 1.3 : 1.
-constexpr int kPipeSides[] = {544, 288, 160, 96};
-constexpr double kPipeTimes[] = {300, 120, 61, 46};
-constexpr int kBatchSides = 4;  // those a batch's problems may get
-constexpr int kServeSides = 4;  // those a request may get
+constexpr int kBatchSides = 4;
+constexpr int kBatchSide[kBatchSides] = {544, 288, 160, 96};
+constexpr int kServeSides = 6;
+constexpr int kServeSide[kServeSides] = {544, 288, 192, 160, 96, 64};
 
-// A round of a tile of level l in us, of a problem `height` rows high (a
-// partial tile takes its share of the steps; a task costs about 8 us besides).
-inline double pipe_tile_us(int height, int l) {
-  const int side = kPipeSides[l];
+// The time of a tile's round in us, a task's 8 beside it.  The rules below
+// compare such times with each other, so that their ratios count.  A batch's
+// are of rounds of sixteen alone on a card, 5.7 : 2.4 : 1.3 : 1 (with every CU
+// busy 440, 169, 88 and 68 us, 6.4 : 2.5 : 1.3 : 1); a request's are those of
+// lone requests to a tolerance of 17 rounds, among them the two that sum
+// exact residuals.
+constexpr double kBatchTimes[kBatchSides] = {300, 120, 61, 46};
+constexpr double kServeTimes[kServeSides] = {422, 152, 104, 76, 52, 43};
+
+// A round of a tile of `side` (a full one takes `us`) of a problem `height`
+// rows high: a partial tile takes its share of the steps.
+inline double pipe_tile_us(double us, int side, int height) {
   const double h = std::min(height, side);
-  return kPipeTimes[l] * (h / 2 + 38) / (side / 2 + 38) + 8;
+  return us * (h / 2 + 38) / (side / 2 + 38) + 8;
 }
 
 // Tile sides of a batch for an engine of groups of waves (blocks[i], those
@@ -56,7 +60,9 @@ inline void pick_blocks(const chm_batch_problem* probs, int n, int n_wg,
     return (double)((probs[i].width + side - 1) / side) *
            ((probs[i].height + side - 1) / side);
   };
-  auto tile_us = [&](int i, int l) { return pipe_tile_us(probs[i].height, l); };
+  auto tile_us = [&](int i, int l) {
+    return pipe_tile_us(kBatchTimes[l], kBatchSide[l], probs[i].height);
+  };
   double work = 0;  // us over all workgroups
   std::vector<Item> heap;
   for (int i = 0; i < n; i++) {
@@ -66,9 +72,9 @@ inline void pick_blocks(const chm_batch_problem* probs, int n, int n_wg,
     }
     int l = 0;  // no side beyond the next one that holds the problem
     const int side = std::max(probs[i].width, probs[i].height);
-    while (l + 1 < kBatchSides && side <= kPipeSides[l + 1]) l++;
-    blocks[i] = kPipeSides[l];
-    work += rounds(i) * tiles(i, kPipeSides[l]) * tile_us(i, l);
+    while (l + 1 < kBatchSides && side <= kBatchSide[l + 1]) l++;
+    blocks[i] = kBatchSide[l];
+    work += rounds(i) * tiles(i, kBatchSide[l]) * tile_us(i, l);
     heap.push_back({rounds(i) * tile_us(i, l), i, l});
   }
   std::make_heap(heap.begin(), heap.end());
@@ -77,13 +83,13 @@ inline void pick_blocks(const chm_batch_problem* probs, int n, int n_wg,
     Item t = heap.back();
     heap.pop_back();
     if (t.level + 1 >= kBatchSides ||
-        tiles(t.i, kPipeSides[t.level + 1]) >= (double)max_tiles)
+        tiles(t.i, kBatchSide[t.level + 1]) >= (double)max_tiles)
       break;  // cannot get shorter
-    const double was = rounds(t.i) * tiles(t.i, kPipeSides[t.level]) *
+    const double was = rounds(t.i) * tiles(t.i, kBatchSide[t.level]) *
                        tile_us(t.i, t.level);
     t.level++;
-    blocks[t.i] = kPipeSides[t.level];
-    work += rounds(t.i) * tiles(t.i, kPipeSides[t.level]) *
+    blocks[t.i] = kBatchSide[t.level];
+    work += rounds(t.i) * tiles(t.i, kBatchSide[t.level]) *
                 tile_us(t.i, t.level) - was;
     t.latency = rounds(t.i) * tile_us(t.i, t.level);
     heap.push_back(t);
@@ -91,25 +97,62 @@ inline void pick_blocks(const chm_batch_problem* probs, int n, int n_wg,
   }
 }
 
-// Tile side of a served request: a finer one where it at least halves the
-// round on this request's share of the workgroups.  It costs 1.4 to 2.1 times
-// as much per cell, which requests that arrive beside this one would miss.
-// (The factor of two was set on one workload, a burst of 24 requests of
-// 256..8192 per side, and others were not tried.)
-inline int serve_block_pipe(int W, int H, int n_wg, int resident,
+// What a server's resident requests take of the card.
+struct ServeLoad {
+  int requests = 0;
+  int64_t tiles = 0;  // tasks of a round of all of them
+  double us = 0;      // workgroup time of such a round
+};
+
+// What a request of H rows in `tiles` tiles of side bs adds to it.
+inline double serve_round_us(int H, int64_t tiles, int bs) {
+  int l = 0;
+  while (l + 1 < kServeSides && kServeSide[l] > bs) l++;
+  return tiles * pipe_tile_us(kServeTimes[l], kServeSide[l], H);
+}
+
+inline double clamp01(double v) { return std::min(1.0, std::max(0.0, v)); }
+
+// Tile side of a served request: the one whose round costs least, in time of
+// - the request: a tile's, or what all residents' tiles take of the card if
+//   that is more (5 % more, by their waits for each other);
+// - a third of a tile's where the card has no room for another such request
+//   beside it, but is not overfilled many times: the last tiles then wait for
+//   a turn of their own;
+// - the residents, whom the request delays by the card time it takes: three
+//   times that as the card fills from half on, and six more as it fills once
+//   more, for the requests that such a load brings besides (of more than
+//   sixteen residents sixteen count);
+// - requests to come: three fifths of that card time.
+// A finer side is over sooner where the card has room for its tiles, but costs
+// 1.4 to 2.1 times as much per cell.  Ms of requests of 300 x 300 x 200 to a
+// tolerance, alone, 6 and 20 at once: 0.90, 0.98, 1.57 (by each request's share
+// of the workgroups, and a finer side only where it halved the round: 1.43,
+// 1.44, 1.49; by the window pass: 1.13, 1.24, 2.22); of 2000 x 2000 x 200
+// alone: 1.95 (2.81; 2.37).  Of 42 bursts of 1..24 drawn requests of up to 7956
+// per side the weights leave none more than 2 % behind the share rule, and take
+// 0.84 of its time on average; with a residents' weight of 1 and 3, 0.81, but
+// one was 8 % behind.
+inline int serve_block_pipe(int W, int H, int n_wg, const ServeLoad& load,
                             int64_t max_tiles) {
-  const int64_t share = std::max<int64_t>(1, n_wg / (1 + resident));
-  int best = kPipeSides[0];
-  double t_best = 0;
+  int best = kServeSide[0];
+  double least = 0;
   for (int l = 0; l < kServeSides; l++) {
-    const int bs = kPipeSides[l];
+    const int bs = kServeSide[l];
     const int64_t tiles = (int64_t)((W + bs - 1) / bs) * ((H + bs - 1) / bs);
     if (l > 0 && tiles >= max_tiles) break;
-    const double t =
-        (double)((tiles + share - 1) / share) * pipe_tile_us(H, l);
-    if (l == 0 || 2 * t <= t_best) {
+    const double us = pipe_tile_us(kServeTimes[l], bs, H);
+    const double card = tiles * us / n_wg;
+    const double full = (double)(load.tiles + tiles) / n_wg;
+    const double twice = (double)(load.tiles + 2 * tiles) / n_wg;
+    const double cost =
+        std::max(us, 1.05 * (load.us / n_wg + card)) + 0.6 * card +
+        clamp01(10 * twice - 9.5) * clamp01(2.5 - twice) * 0.35 * us +
+        (3 * clamp01(2 * full - 1) + 6 * clamp01(2 * full - 2)) *
+            std::min(load.requests, 16) * card;
+    if (l == 0 || cost < least) {
       best = bs;
-      t_best = t;
+      least = cost;
     }
   }
   return best;

@@ -23,9 +23,19 @@ extern "C" void batch_sides(const int* probs, int n, int n_wg, long max_tiles,
   chm::eng::pick_blocks(p.data(), n, n_wg, max_tiles, b);
   for (int i = 0; i < n; i++) sides[i] = b[i];
 }
-extern "C" int serve_side(int w, int h, int n_wg, int resident,
-                          long max_tiles) {
-  return chm::eng::serve_block_pipe(w, h, n_wg, resident, max_tiles);
+// requests in order: the side of each with all before it resident
+extern "C" void serve_sides(const int* wh, int n, int n_wg, long max_tiles,
+                            int* sides) {
+  chm::eng::ServeLoad load;
+  for (int i = 0; i < n; i++) {
+    const int w = wh[2 * i], h = wh[2 * i + 1];
+    const int bs = chm::eng::serve_block_pipe(w, h, n_wg, load, max_tiles);
+    const long tiles = (long)((w + bs - 1) / bs) * ((h + bs - 1) / bs);
+    load.requests++;
+    load.tiles += tiles;
+    load.us += chm::eng::serve_round_us(h, tiles, bs);
+    sides[i] = bs;
+  }
 }
 """
 CUS, MAX_TILES = 256, 1 << 18
@@ -41,14 +51,20 @@ def rules(tmp_path_factory):
     L = ctypes.CDLL(str(d / "r.so"))
     L.batch_sides.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
                               ctypes.c_long, ctypes.c_void_p]
-    L.serve_side.argtypes = [ctypes.c_int] * 4 + [ctypes.c_long]
+    L.serve_sides.argtypes = L.batch_sides.argtypes
 
     def batch(probs, n_wg=CUS, max_tiles=MAX_TILES):
         flat = (ctypes.c_int * (5 * len(probs)))(*[v for p in probs for v in p])
         out = (ctypes.c_int * len(probs))()
         L.batch_sides(flat, len(probs), n_wg, max_tiles, out)
         return list(out)
-    return batch, L.serve_side
+
+    def serve(wh, n_wg=CUS, max_tiles=MAX_TILES):
+        flat = (ctypes.c_int * (2 * len(wh)))(*[v for p in wh for v in p])
+        out = (ctypes.c_int * len(wh))()
+        L.serve_sides(flat, len(wh), n_wg, max_tiles, out)
+        return list(out)
+    return batch, serve
 
 
 def test_caps_do_not_tell_where_a_tolerance_stops(rules):
@@ -79,3 +95,37 @@ def test_given_sides_and_the_tile_limit(rules):
     # 5000 x 5000 in tiles of 96 would be 2809
     side, = batch([(5000, 5000, 500, 0, 0)], n_wg=100000, max_tiles=2000)
     assert side == 160
+
+
+def test_a_lone_request_is_spread(rules):
+    # small ones in the finest tiles, larger ones in finer ones than 288 as
+    # long as the card has room, the largest in few turns of the card
+    _, serve = rules
+    for side, want in [(100, 64), (300, 64), (600, 64), (1000, 96), (2000, 192),
+                       (2048, 192), (3000, 160), (4000, 288), (6000, 288),
+                       (8000, 544), (20000, 544)]:
+        assert serve([(side, side)]) == [want], side
+    assert max(serve([(3000, 50)]) + serve([(50, 3000)]) + serve([(9, 9)])) <= 96
+
+
+def test_a_few_small_requests_are_spread_too(rules):
+    _, serve = rules
+    assert serve([(300, 300)] * 6) == [64] * 6
+    assert set(serve([(148, 148)] * 30)) <= {64, 96}
+
+
+def test_sides_grow_with_the_load(rules):
+    _, serve = rules
+    for side in (300, 600, 1000, 2000, 5000):
+        got = serve([(side, side)] * 60)
+        assert got[0] == min(got) and got[-1] == max(got) >= 160
+    assert set(serve([(2000, 2000)] * 60)[30:]) == {544}
+    # a tile of 300 x 300 would make its round three times as long as four of
+    # 160: not even then
+    assert serve([(300, 300)] * 100)[-1] == 160
+
+
+def test_request_tile_limit(rules):
+    _, serve = rules
+    assert serve([(2000, 2000)], max_tiles=100) == [288]
+    assert serve([(2000, 2000)], max_tiles=1) == [544]
