@@ -23,33 +23,32 @@ __host__ __device__ inline int lanes_log2(int cols, int threads) {
 
 // Thread t of workgroup wg of n_wg, of `threads` threads each (a power of
 // two).  A workgroup takes a row at a time, or several of a region narrower
-// than it is.  Where that leaves workgroups over, each row is cut into as many
-// interleaved parts as there are workgroups for, down to four cells a thread.
-// (A whole row to a workgroup at any shape kept one busy on 1 x 2.7M
-// cells and sixteen on 16 x 1M: a no-alloc solve of 2 sweeps of 1 x 2.7M took
-// 5117 us, now 160; the hash of 16 x 1M 1330, now 60; of 1M x 16, where 16 of
-// 256 lanes had a cell, 424, now 64.  Grids of 2000 x 2000 are as fast.)
+// than it is.  Of fewer rows than two turns of the workgroups each is cut into
+// interleaved parts, down to four cells a thread, and each part has a team of
+// workgroups, so that all have about the same to do.  (Whole rows only kept one
+// workgroup busy on 1 x 2.7M cells, sixteen on 16 x 1M and half of them on
+// 526 x 70506: a no-alloc solve of 2 sweeps of the first took 5117 us, now 160;
+// the hash of the others 1330, now 60, and 183, now 120; of 1M x 16, where 16
+// of 256 lanes had a cell, 424, now 62.  Grids of 2000 x 2000 are as fast.)
 __host__ __device__ inline CellShare cell_share(int rows, int cols, int wg,
                                                 int n_wg, int threads, int t) {
   if (rows <= 0 || cols <= 0) return {rows, 1, cols, 1};
   const int lg = lanes_log2(cols, threads), lanes = 1 << lg;
   const int pg = lanes_log2(threads, threads) - lg;  // 2^pg rows at a time
   const int groups = (rows + (1 << pg) - 1) >> pg;
-  CellShare s;
-  int segs = 1, group = wg, seg = 0;
-  if (groups < n_wg) {
-    const int most = cols >> (lg + kCellsLog2);
-    if (most > 1) {
-      const int have = n_wg / groups;
-      segs = have < most ? have : most;
-    }
-    if (wg >= groups) {
-      seg = wg / groups;
-      group = seg < segs ? wg - seg * groups : groups;  // (none left for it)
-    }
+  int segs = 1, team = n_wg, seg = 0, of_team = wg;
+  const int most = cols >> (lg + kCellsLog2);
+  if (groups < 2 * n_wg && most > 1) {
+    const int want = 8 * n_wg / groups;
+    segs = want < most ? want : most;
+    segs = segs < n_wg ? segs : n_wg;
+    team = n_wg / segs;
+    seg = wg / team;
+    of_team = seg < segs ? wg - seg * team : groups;  // (left over)
   }
-  s.row = (group << pg) + (t >> lg);
-  s.row_step = (groups < n_wg ? groups : n_wg) << pg;
+  CellShare s;
+  s.row = (of_team << pg) + (t >> lg);
+  s.row_step = team << pg;
   s.col = (seg << lg) + (t & (lanes - 1));
   s.col_step = segs << lg;
   return s;
