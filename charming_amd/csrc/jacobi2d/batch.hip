@@ -2039,8 +2039,8 @@ int chm_jacobi2d_server_submit(void* handle, const chm_batch_problem* pb,
   int block = s->block;
   if (engine && pb->block <= 0 && block <= 0)
     block = s->e.threads == kPipeThreads
-                ? serve_block_pipe(pb->width, pb->height, s->e.d.n_wg, s->load,
-                                   kMaxTiles)
+                ? serve_block_pipe(pb->width, pb->height, pb->iters,
+                                   s->e.d.n_wg, s->load, kMaxTiles)
                 : serve_block(pb->width, pb->height, s->e.d.n_wg,
                               (int)s->live.size(),
                               jac::window_out_cols(
@@ -2069,9 +2069,9 @@ int chm_jacobi2d_server_submit(void* handle, const chm_batch_problem* pb,
   r.slot = s->free_slots.back();
   s->free_slots.pop_back();
   const int64_t tiles = (int64_t)r.tr * r.tc;
-  const Server::Live& l = s->live[r.ticket] =
-      Server::Live{off,     bytes, r.slot,
-                   now_s(), tiles, serve_round_us(r.H, tiles, r.bs)};
+  const Server::Live& l = s->live[r.ticket] = Server::Live{
+      off,     bytes, r.slot,
+      now_s(), tiles, serve_round_us(r.W, r.H, pb->iters, tiles, r.bs)};
   s->load.requests++;
   s->load.tiles += l.tiles;
   s->load.us += l.round_us;

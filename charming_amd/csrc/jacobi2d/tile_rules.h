@@ -21,10 +21,9 @@ constexpr int kServeSide[kServeSides] = {544, 288, 192, 160, 96, 64};
 // compare such times with each other, so that their ratios count.  A batch's
 // are of rounds of sixteen alone on a card, 5.7 : 2.4 : 1.3 : 1 (with every CU
 // busy 440, 169, 88 and 68 us, 6.4 : 2.5 : 1.3 : 1); a request's are those of
-// lone requests to a tolerance of 17 rounds, among them the two that sum
-// exact residuals.
+// lone requests to a tolerance of 17 rounds, less what its tiles cost once.
 constexpr double kBatchTimes[kBatchSides] = {300, 120, 61, 46};
-constexpr double kServeTimes[kServeSides] = {422, 152, 104, 76, 52, 43};
+constexpr double kServeTimes[kServeSides] = {337, 130, 93, 69, 49, 42};
 
 // A round of a tile of `side` (a full one takes `us`) of a problem `height`
 // rows high: a partial tile takes its share of the steps.
@@ -97,6 +96,16 @@ inline void pick_blocks(const chm_batch_problem* probs, int n, int n_wg,
   }
 }
 
+// The same for a request of `iters` sweeps, with its share of what a tile takes
+// once: to be seeded and hashed and for the sums of exact residuals, 4.9 ns a
+// cell (of one sweep, 11 requests of 500 x 500 took 0.53 ms in tiles of 288, now
+// 0.32 in tiles of 64 and 96).
+inline double serve_tile_us(int l, int W, int H, int iters) {
+  const int side = kServeSide[l], rounds = (iters + 15) / 16;
+  return pipe_tile_us(kServeTimes[l], side, H) +
+         4.9e-3 * std::min(W, side) * std::min(H, side) / std::max(1, rounds);
+}
+
 // What a server's resident requests take of the card.
 struct ServeLoad {
   int requests = 0;
@@ -104,11 +113,11 @@ struct ServeLoad {
   double us = 0;      // workgroup time of such a round
 };
 
-// What a request of H rows in `tiles` tiles of side bs adds to it.
-inline double serve_round_us(int H, int64_t tiles, int bs) {
+// What a request in `tiles` tiles of side bs adds to it.
+inline double serve_round_us(int W, int H, int iters, int64_t tiles, int bs) {
   int l = 0;
   while (l + 1 < kServeSides && kServeSide[l] > bs) l++;
-  return tiles * pipe_tile_us(kServeTimes[l], kServeSide[l], H);
+  return tiles * serve_tile_us(l, W, H, iters);
 }
 
 inline double clamp01(double v) { return std::min(1.0, std::max(0.0, v)); }
@@ -133,15 +142,15 @@ inline double clamp01(double v) { return std::min(1.0, std::max(0.0, v)); }
 // per side the weights leave none more than 2 % behind the share rule, and take
 // 0.84 of its time on average; with a residents' weight of 1 and 3, 0.81, but
 // one was 8 % behind.
-inline int serve_block_pipe(int W, int H, int n_wg, const ServeLoad& load,
-                            int64_t max_tiles) {
+inline int serve_block_pipe(int W, int H, int iters, int n_wg,
+                            const ServeLoad& load, int64_t max_tiles) {
   int best = kServeSide[0];
   double least = 0;
   for (int l = 0; l < kServeSides; l++) {
     const int bs = kServeSide[l];
     const int64_t tiles = (int64_t)((W + bs - 1) / bs) * ((H + bs - 1) / bs);
     if (l > 0 && tiles >= max_tiles) break;
-    const double us = pipe_tile_us(kServeTimes[l], bs, H);
+    const double us = serve_tile_us(l, W, H, iters);
     const double card = tiles * us / n_wg;
     const double full = (double)(load.tiles + tiles) / n_wg;
     const double twice = (double)(load.tiles + 2 * tiles) / n_wg;

@@ -25,15 +25,16 @@ extern "C" void batch_sides(const int* probs, int n, int n_wg, long max_tiles,
 }
 // requests in order: the side of each with all before it resident
 extern "C" void serve_sides(const int* wh, int n, int n_wg, long max_tiles,
-                            int* sides) {
+                            int* sides, int iters) {
   chm::eng::ServeLoad load;
   for (int i = 0; i < n; i++) {
     const int w = wh[2 * i], h = wh[2 * i + 1];
-    const int bs = chm::eng::serve_block_pipe(w, h, n_wg, load, max_tiles);
+    const int bs =
+        chm::eng::serve_block_pipe(w, h, iters, n_wg, load, max_tiles);
     const long tiles = (long)((w + bs - 1) / bs) * ((h + bs - 1) / bs);
     load.requests++;
     load.tiles += tiles;
-    load.us += chm::eng::serve_round_us(h, tiles, bs);
+    load.us += chm::eng::serve_round_us(w, h, iters, tiles, bs);
     sides[i] = bs;
   }
 }
@@ -51,7 +52,7 @@ def rules(tmp_path_factory):
     L = ctypes.CDLL(str(d / "r.so"))
     L.batch_sides.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
                               ctypes.c_long, ctypes.c_void_p]
-    L.serve_sides.argtypes = L.batch_sides.argtypes
+    L.serve_sides.argtypes = L.batch_sides.argtypes + [ctypes.c_int]
 
     def batch(probs, n_wg=CUS, max_tiles=MAX_TILES):
         flat = (ctypes.c_int * (5 * len(probs)))(*[v for p in probs for v in p])
@@ -59,10 +60,10 @@ def rules(tmp_path_factory):
         L.batch_sides(flat, len(probs), n_wg, max_tiles, out)
         return list(out)
 
-    def serve(wh, n_wg=CUS, max_tiles=MAX_TILES):
+    def serve(wh, n_wg=CUS, max_tiles=MAX_TILES, iters=1500):
         flat = (ctypes.c_int * (2 * len(wh)))(*[v for p in wh for v in p])
         out = (ctypes.c_int * len(wh))()
-        L.serve_sides(flat, len(wh), n_wg, max_tiles, out)
+        L.serve_sides(flat, len(wh), n_wg, max_tiles, out, iters)
         return list(out)
     return batch, serve
 
@@ -105,12 +106,12 @@ def test_a_lone_request_is_spread(rules):
                        (2048, 192), (3000, 160), (4000, 288), (6000, 288),
                        (8000, 544), (20000, 544)]:
         assert serve([(side, side)]) == [want], side
-    assert max(serve([(3000, 50)]) + serve([(50, 3000)]) + serve([(9, 9)])) <= 96
+    assert max(serve([(3000, 50)]) + serve([(50, 3000)]) + serve([(9, 9)])) <= 160
 
 
 def test_a_few_small_requests_are_spread_too(rules):
     _, serve = rules
-    assert serve([(300, 300)] * 6) == [64] * 6
+    assert set(serve([(300, 300)] * 6)) <= {64, 96}
     assert set(serve([(148, 148)] * 30)) <= {64, 96}
 
 
@@ -123,6 +124,14 @@ def test_sides_grow_with_the_load(rules):
     # a tile of 300 x 300 would make its round three times as long as four of
     # 160: not even then
     assert serve([(300, 300)] * 100)[-1] == 160
+
+
+def test_few_sweeps_take_finer_tiles(rules):
+    # to seed and hash a tile of 288 takes as long as three of its rounds
+    _, serve = rules
+    few = serve([(500, 500)] * 11, iters=5)
+    many = serve([(500, 500)] * 11, iters=1500)
+    assert max(few) <= 96 and all(f <= m for f, m in zip(few, many))
 
 
 def test_request_tile_limit(rules):
