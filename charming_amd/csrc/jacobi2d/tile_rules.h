@@ -99,7 +99,7 @@ inline void pick_blocks(const chm_batch_problem* probs, int n, int n_wg,
 // The same for a request of `iters` sweeps, with its share of what a tile takes
 // once: to be seeded and hashed and for the sums of exact residuals, 4.9 ns a
 // cell (of one sweep, 11 requests of 500 x 500 took 0.53 ms in tiles of 288, now
-// 0.32 in tiles of 64 and 96).
+// 0.32 in tiles of 64, 96 and 192).
 inline double serve_tile_us(int l, int W, int H, int iters) {
   const int side = kServeSide[l], rounds = (iters + 15) / 16;
   return pipe_tile_us(kServeTimes[l], side, H) +
