@@ -2,6 +2,7 @@
 // the kernels that touch each cell once (fill, hash, residual), with no
 // division per cell.
 #pragma once
+#include <math.h>
 
 namespace chm {
 namespace jac {
@@ -38,7 +39,11 @@ __host__ __device__ inline CellShare cell_share(int rows, int cols, int wg,
   const int groups = (rows + (1 << pg) - 1) >> pg;
   int segs = 1, team = n_wg, seg = 0, of_team = wg;
   const int most = cols >> (lg + kCellsLog2);
-  if (groups < 2 * n_wg && most > 1) {
+  // (an eighth of the last turn's workgroups may be idle: cut, 316 rows for
+  // 316 workgroups would be eight turns of a seventh of a row)
+  const bool full = groups <= n_wg ? groups > n_wg - n_wg / 8
+                                   : groups > 2 * n_wg - n_wg / 8;
+  if (!full && most > 1) {
     const int want = 8 * n_wg / groups;
     segs = want < most ? want : most;
     segs = segs < n_wg ? segs : n_wg;
@@ -62,6 +67,32 @@ inline int cell_wgs(int rows, int cols, int threads, int most) {
   const long long n =
       (long long)((rows + per - 1) / per) * (segs < 1 ? 1 : segs);
   return (int)(n < most ? n : most);
+}
+
+// Workgroups for a sum over the region, whose workgroups each end in one or two
+// atomics on one cache line.  Those are done one after another, 9 ns each, and
+// a thread's cells are too, so n workgroups take a cells / n + b n: least at a
+// multiple of sqrt(cells), of which 1 / c is what runs of 64..1024 workgroups on
+// 19 shapes gave: c 2.5 for the hash and the residual (one atomic), 5 for the
+// hash that counts its workgroups besides.  2800 x 500: 256 workgroups take
+// 30.1 and 14.6 us, 1024 37.0 and 30.8; 2800 x 2800: 54 and 39 us with 384, 45
+// and 40 with 1024, which is the most: four a CU.
+inline int sum_wgs(int rows, int cols, int threads, double c) {
+  int n = 1024;
+  const double best = sqrt((double)rows * (double)cols) / c;
+  if (best < n) {
+    n = best < 64 ? 64 : (int)best;
+    // whole turns of whole rows where they are about as many (7627 x 316: 17.8
+    // us with 316 workgroups, 19.4 with 310)
+    const int per = threads >> lanes_log2(cols, threads);
+    const int groups = rows / per + (rows % per > 0);
+    if (5LL * groups >= 3 * n) {
+      const int turns = (int)(((long long)2 * groups + n) / (2 * n));
+      n = (groups - 1) / turns + 1;
+    }
+  }
+  n = cell_wgs(rows, cols, threads, n);
+  return n < 1 ? 1 : n > 1024 ? 1024 : n;  // (an empty region's sum is 0)
 }
 
 }  // namespace jac

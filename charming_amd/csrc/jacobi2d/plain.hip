@@ -321,11 +321,12 @@ static int plain_solve(Handle* h, chm_jacobi_result* res) {
     res->iters_done = iters;
     res->launches = launches;
     CHM_TRY_HIP(hipMemsetAsync(h->d_acc, 0, 4 * sizeof(uint64_t), h->stream));
+    const int sums = sum_wgs(h->H, h->W, 256, 2.5);
     if (iters > 0)
-      residual_global_kernel<<<1024, 256, 0, h->stream>>>(
+      residual_global_kernel<<<sums, 256, 0, h->stream>>>(
           h->grid[h->cur], h->grid[h->cur ^ 1], h->W, h->H, h->P,
           h->d_acc + 1);
-    hash_global_kernel<<<1024, 256, 0, h->stream>>>(
+    hash_global_kernel<<<sums, 256, 0, h->stream>>>(
         h->grid[h->cur], h->P, 1, h->H + 1, 1, h->W + 1, h->d_acc);
     CHM_TRY_HIP(hipGetLastError());
     uint64_t acc[4];
@@ -563,7 +564,7 @@ static int solve_noalloc(double* grid, int W, int H, int iters,
                            L.n_tiles, L.n_blocks);
     }
   }
-  end_noalloc_kernel<<<cell_wgs(H, W, 256, 1024), 256, 0, stream>>>(
+  end_noalloc_kernel<<<sum_wgs(H, W, 256, 5), 256, 0, stream>>>(
       g[cur], cur ? grid : nullptr, W, H, P, acc, out3);
   CHM_TRY_HIP(hipGetLastError());
   return CHM_OK;
@@ -741,8 +742,9 @@ int chm_jacobi2d_hash_region(void* handle, int r0, int r1, int c0, int c1,
   if (h->form == CHM_FORM_PERSISTENT)
     return persistent_hash_region(h, r0, r1, c0, c1, hash);
   CHM_TRY_HIP(hipMemsetAsync(h->d_acc, 0, sizeof(uint64_t), h->stream));
-  hash_global_kernel<<<1024, 256, 0, h->stream>>>(h->grid[h->cur], h->P, r0,
-                                                  r1, c0, c1, h->d_acc);
+  hash_global_kernel<<<sum_wgs(r1 - r0, c1 - c0, 256, 2.5), 256, 0,
+                       h->stream>>>(
+      h->grid[h->cur], h->P, r0, r1, c0, c1, h->d_acc);
   CHM_TRY_HIP(hipGetLastError());
   CHM_TRY_HIP(hipMemcpyAsync(hash, h->d_acc, sizeof(uint64_t),
                              hipMemcpyDeviceToHost, h->stream));

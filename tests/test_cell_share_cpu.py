@@ -81,3 +81,39 @@ def test_empty_regions_take_no_cell(exe):
         [exe] + [str(v) for s in ((0, 7), (7, 0)) for v in (*s, 64, 256)],
         text=True).split()
     assert out == ["1", "0", "0"] * 2
+
+
+SUM_SRC = r"""
+#define __host__
+#define __device__
+#include "cell_share.h"
+#include <stdio.h>
+#include <stdlib.h>
+int main(int argc, char** argv) {
+  for (int a = 1; a + 2 < argc; a += 3)
+    printf("%d\n", chm::jac::sum_wgs(atoi(argv[a]), atoi(argv[a + 1]), 256,
+                                     atof(argv[a + 2])));
+}
+"""
+
+
+def test_workgroups_of_a_sum(tmp_path):
+    """At least one, at most 1024, no more than have a cell; and where rows
+    are few, not so many that their atomics outlast the cells."""
+    (tmp_path / "main.cpp").write_text(SUM_SRC)
+    exe = str(tmp_path / "main")
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-I", CSRC,
+                           str(tmp_path / "main.cpp"), "-o", exe])
+    shapes = SHAPES + [(0, 7), (7, 0), (16384, 16384), (1, 1 << 30),
+                       (1 << 30, 1)]
+    out = subprocess.check_output(
+        [exe] + [str(v) for s in shapes for c in (2.5, 5) for v in (*s, c)],
+        text=True).split()
+    for (rows, cols), a, b in zip(shapes, out[::2], out[1::2]):
+        for n in (int(a), int(b)):
+            assert 1 <= n <= 1024, (rows, cols, n)
+            assert n <= max(1, rows * cols), (rows, cols, n)
+    few = subprocess.check_output(
+        [exe] + "500 2800 2.5 500 2800 5 200 2800 2.5 200 2800 5".split(),
+        text=True).split()
+    assert all(int(n) <= 512 for n in few), few
