@@ -29,7 +29,7 @@ __host__ __device__ inline int lanes_log2(int cols, int threads) {
 // workgroups, so that all have about the same to do.  (Whole rows only kept one
 // workgroup busy on 1 x 2.7M cells, sixteen on 16 x 1M and half of them on
 // 526 x 70506: a no-alloc solve of 2 sweeps of the first took 5117 us, now 160;
-// the hash of the others 1330, now 60, and 183, now 120; of 1M x 16, where 16
+// the hash of the others 1330, now 58, and 183, now 120; of 1M x 16, where 16
 // of 256 lanes had a cell, 424, now 62.  Grids of 2000 x 2000 are as fast.)
 __host__ __device__ inline CellShare cell_share(int rows, int cols, int wg,
                                                 int n_wg, int threads, int t) {
@@ -74,7 +74,7 @@ inline int cell_wgs(int rows, int cols, int threads, int most) {
 // a thread's cells are too, so n workgroups take a cells / n + b n: least at a
 // multiple of sqrt(cells), of which 1 / c is what runs of 64..1024 workgroups on
 // 19 shapes gave: c 2.5 for the hash and the residual (one atomic), 5 for the
-// hash that counts its workgroups besides.  2800 x 500: 256 workgroups take
+// hash that counts its workgroups besides.  500 x 2800: 256 workgroups take
 // 30.1 and 14.6 us, 1024 37.0 and 30.8; 2800 x 2800: 54 and 39 us with 384, 45
 // and 40 with 1024, which is the most: four a CU.
 inline int sum_wgs(int rows, int cols, int threads, double c) {
@@ -82,7 +82,7 @@ inline int sum_wgs(int rows, int cols, int threads, double c) {
   const double best = sqrt((double)rows * (double)cols) / c;
   if (best < n) {
     n = best < 64 ? 64 : (int)best;
-    // whole turns of whole rows where they are about as many (7627 x 316: 17.8
+    // whole turns of whole rows where they are about as many (316 x 7627: 17.8
     // us with 316 workgroups, 19.4 with 310)
     const int per = threads >> lanes_log2(cols, threads);
     const int groups = rows / per + (rows % per > 0);

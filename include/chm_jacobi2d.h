@@ -259,9 +259,11 @@ typedef struct chm_server_config {
   int max_active;      /* requests resident at once (0 = 4096) */
   int wg_threads, block, panel_chunks, rows_in_flight; /* as chm_batch_config
                           (wg_threads 0 = 512: tolerance rounds of twelve);
-                          block 0 = by load: tiles as large as a request's
-                          share of the workgroups, 1 / (1 + resident
-                          requests), allows */
+                          block 0 = by load: at 512 threads the tiles whose
+                          rounds cost the request and the residents least,
+                          by the room that these leave on the card; else as
+                          large as a request's share of the workgroups,
+                          1 / (1 + resident requests), allows */
 } chm_server_config;
 
 typedef struct chm_server_completion {
