@@ -437,7 +437,7 @@ __global__ void end_noalloc_kernel(const double* g, double* copy, int W, int H,
 // 4 NST sweeps of a whole grid in one launch: a tile of tw x th cells per
 // workgroup (one per CU), swept by two groups of four waves (pipeline.h).
 // A launch per sweep was bound by its launch and by a few waves walking long
-// bands: 1021 x 683 x 100 took 5.28 ms, now 0.21; 2800 x 2800 x 200 16.3 ms,
+// bands: 1021 x 683 x 100 took 5.28 ms, now 0.20; 2800 x 2800 x 200 16.3 ms,
 // now 1.04 (5 TB/s of the caches would allow 0.3; the tiles' margins and the
 // filling of their pipelines double the arithmetic); 64 x 64 x 10 345 us,
 // now 34, in six launches.
