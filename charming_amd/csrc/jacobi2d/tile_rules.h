@@ -106,6 +106,20 @@ inline double serve_tile_us(int l, int W, int H, int iters) {
          4.9e-3 * std::min(W, side) * std::min(H, side) / std::max(1, rounds);
 }
 
+// The workgroup time of a round of the request: its tiles, those at its right
+// and lower edge in their own sizes (a row of a window costs by the columns per
+// lane that hold it, 3, 5 or 9).
+inline double serve_request_us(int l, int W, int H, int iters) {
+  const int side = kServeSide[l], rounds = std::max(1, (iters + 15) / 16);
+  auto step = [](int w) { return w <= 160 ? 0.585 : w <= 288 ? 0.71 : 1.09; };
+  // all columns' steps of one row of the request, and all rows' of one column
+  const int cw = W / side, rw = W % side, ch = H / side, rh = H % side;
+  const double row = cw * step(side) + (rw ? step(rw) : 0);
+  const double col = ch * (side / 2.0 + 38) + (rh ? rh / 2.0 + 38 : 0);
+  return row * col + 8.0 * (cw + (rw > 0)) * (ch + (rh > 0)) +
+         4.9e-3 * W * H / rounds;
+}
+
 // What a server's resident requests take of the card.
 struct ServeLoad {
   int requests = 0;
@@ -128,10 +142,12 @@ inline double clamp01(double v) { return std::min(1.0, std::max(0.0, v)); }
 // - a third of a tile's where the card has no room for another such request
 //   beside it, but is not overfilled many times: the last tiles then wait for
 //   a turn of their own;
-// - the residents, whom the request delays by the card time it takes: three
-//   times that as the card fills from half on, and six more as it fills once
-//   more, for the requests that such a load brings besides (of more than
-//   sixteen residents sixteen count);
+// - the residents, whom the request delays by the card time it takes (partial
+//   tiles at their own sizes: counted full, a request a little wider than 544
+//   went to tiles of 288, 250.9 requests a second of a saturated stream, now
+//   253.9): three times that as the card fills from half on, and six more as it
+//   fills once more, for the requests that such a load brings besides (of more
+//   than sixteen residents sixteen count);
 // - requests to come: three fifths of that card time.
 // A finer side is over sooner where the card has room for its tiles, but costs
 // 1.4 to 2.1 times as much per cell.  Ms of requests of 300 x 300 x 200 to a
@@ -152,13 +168,14 @@ inline int serve_block_pipe(int W, int H, int iters, int n_wg,
     if (l > 0 && tiles >= max_tiles) break;
     const double us = serve_tile_us(l, W, H, iters);
     const double card = tiles * us / n_wg;
+    const double delay = serve_request_us(l, W, H, iters) / n_wg;
     const double full = (double)(load.tiles + tiles) / n_wg;
     const double twice = (double)(load.tiles + 2 * tiles) / n_wg;
     const double cost =
         std::max(us, 1.05 * (load.us / n_wg + card)) + 0.6 * card +
         clamp01(10 * twice - 9.5) * clamp01(2.5 - twice) * 0.35 * us +
         (3 * clamp01(2 * full - 1) + 6 * clamp01(2 * full - 2)) *
-            std::min(load.requests, 16) * card;
+            std::min(load.requests, 16) * delay;
     if (l == 0 || cost < least) {
       best = bs;
       least = cost;

@@ -138,3 +138,12 @@ def test_request_tile_limit(rules):
     _, serve = rules
     assert serve([(2000, 2000)], max_tiles=100) == [288]
     assert serve([(2000, 2000)], max_tiles=1) == [544]
+
+
+def test_partial_tiles_cost_their_own_size(rules):
+    # with the card full what counts is the work: two tiles of 544 where the
+    # second is a strip cost less than three of 288
+    _, serve = rules
+    full = [(2000, 2000)] * 60
+    for wh in [(584, 1329), (597, 283), (668, 1210), (740, 571), (3323, 1102)]:
+        assert serve(full + [wh])[-1] == 544, wh
