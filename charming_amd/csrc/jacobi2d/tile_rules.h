@@ -157,7 +157,10 @@ inline double clamp01(double v) { return std::min(1.0, std::max(0.0, v)); }
 // alone: 1.95 (2.81; 2.37).  Of 42 bursts of 1..24 drawn requests of up to 7956
 // per side the weights leave none more than 2 % behind the share rule, and take
 // 0.84 of its time on average; with a residents' weight of 1 and 3, 0.81, but
-// one was 8 % behind.
+// one was 8 % behind.  Requests of one size submitted at once are where the
+// greedy choice costs: the first take tiles that the next have no room beside.
+// Of 80 bursts of 1 to 20 such the rule takes 0.83 of the share rule's time, but
+// 30 are more than 3 % slower (2 of 959 x 959 x 12: 292 us, 182 in tiles of 96).
 inline int serve_block_pipe(int W, int H, int iters, int n_wg,
                             const ServeLoad& load, int64_t max_tiles) {
   int best = kServeSide[0];
